@@ -366,6 +366,7 @@ bool build_taps(const MonitorPlan& mp, int slot0, int t_rel0, int esz, TapSet* o
     for (int q = 0; q < m.n_terms; ++q) {
       const mt_dft_term& tm = m.term[q];
       if (tm.line < 1 || tm.line > 4 || out->n >= kMaxTaps) return false;
+      if (tm.field >= 3 && tm.b) return false;  // D values are not averaged in a tile
       Tap& t = out->t[out->n++];
       t.field = tm.field;
       t.line = tm.line;

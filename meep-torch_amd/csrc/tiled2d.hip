@@ -3,8 +3,8 @@
 //
 // A workgroup owns a TX x TY block of the (i, j) cell lattice.  It loads the
 // block plus a halo (NS+1 cells on the low sides, NS on the high sides) of
-// the evolving fields into LDS, advances NS steps there, and writes back only
-// the cells it owns.  Per half-step the stencil reaches one cell (D/E halves
+// the evolving fields, advances NS steps on chip, and writes back only the
+// cells it owns.  Per half-step the stencil reaches one cell (D/E halves
 // towards lower indices, H/B halves towards higher ones), so after NS steps
 // every owned cell, and the one row/column below it that averaged H monitor
 // samples need, is exact.  Halo cells are recomputed redundantly; cells whose
@@ -12,14 +12,24 @@
 // an owned cell.  Reads come from one set of global buffers and writes go to
 // the other (ping-pong), so tiles never see each other's partial results.
 //
+// Thread mapping: a thread owns one column lj of the region and every
+// ROWS-th row of it (rows l0, l0 + ROWS, ...), the same cells in every
+// sub-step.  All of a cell's values live in its thread's registers (fields,
+// D, eps, CPML memory); the LDS holds only the copies that neighbours and
+// monitor taps read.  The column's CPML profile values are per-thread
+// constants in registers, the rows' come from a small LDS table, so the
+// sub-step loop touches no global memory.  (Before, a thread's cells were a
+// flat stride through the region: every half-step recomputed each cell's
+// row, column and bounds and read the CPML profiles from global memory.
+// TE 2048^2, 16x64x4: 25.7 -> 23.4 us per step; the CPML ring of a 256^2 TM
+// grid, where that latency was the whole launch, 7.9 -> 3.9 us per step.)
+//
 // Arithmetic per cell is the per-half-step kernels' (yee2d.hip), op for op,
 // so results are bit-identical to them and to the reference's FP32 stepper.
-// Tiles whose halo touches a CPML shell also run the four psi recursions
-// (template PML = true), with each cell's psi values in the registers of
-// the thread that updates it (the recursion is pointwise, so psi needs no
-// LDS); interior tiles carry none and run in a separate launch.  Monitor samples are taken inside the tile after each step by the
-// tile that owns the sampled cell and written to the staging ring consumed by
-// the DFT flush (dft.hip).
+// Tiles whose region touches a CPML shell also run the four psi recursions
+// (template PML = true); interior tiles carry none.  Monitor samples are
+// taken inside the tile after each step by the tile that owns the sampled
+// cell and written to the staging ring consumed by the DFT flush (dft.hip).
 #include <hip/hip_runtime.h>
 
 #include "common.h"
@@ -30,20 +40,51 @@
 namespace mt {
 namespace {
 
-// Threads per tile workgroup.  TM tiles run 1024 threads (3-6 cells per
-// thread at NS = 4): the TM step is light and the design loops' grids are
-// small, so more waves per tile shorten each launch.  TE interior tiles run
-// 512: on 2048^2 the interior TE launch is arithmetic-bound and 1024-thread
-// interior tiles measured slower (98 -> 123 us per launch).
-constexpr int BLK_TM = 1024;
-// TE: 512 threads for interior tiles; CPML ring tiles (few, each carrying
-// the psi recursions, so the ring launch is one latency chain per CU) run
-// 1024 threads, which shortens each thread's share of a tile.
-constexpr int te_block(bool pml) { return pml ? 1024 : 512; }
-
 template <typename T>
 __device__ __forceinline__ T dget(const T* p, long long idx, bool ok) {
   return ok ? p[idx] : T(0);
+}
+
+// LDS region of a TX x TY x NS tile and its thread mapping for at most MAXB
+// threads: PER rows per thread, ROWS rows per pass, BLK threads.
+template <int TX, int TY, int NS, int MAXB>
+struct Shape {
+  static constexpr int RX = TX + 2 * NS + 1, RY = TY + 2 * NS + 1, RC = RX * RY;
+  static constexpr int PASSES = (RX + MAXB / RY - 1) / (MAXB / RY);
+  static constexpr int ROWS = (RX + PASSES - 1) / PASSES;
+  static constexpr int PER = (RX + ROWS - 1) / ROWS;
+  static constexpr int STR = ROWS * RY;
+  static constexpr int BLK = (STR + 63) / 64 * 64;
+  static_assert(MAXB >= RY && BLK <= 1024, "tile rows must fit a workgroup");
+};
+
+// Quotients ax(u) / dx and ay(u) / dx of one half-step, checked together:
+// each takes div_c's fast sequence and records its dividend's exponent; a
+// lane for which some dividend falls outside the verified range (or a
+// divisor without a verified reciprocal, rdx = 0) redoes its quotients with
+// IEEE division, from dividends formed again (the LDS values they read do not
+// change within a half-step).  FP64 always divides.
+template <typename T, int PER, typename FX, typename FY>
+__device__ __forceinline__ void step_quots(T dx, T rdx, FX ax, FY ay, T (&qx)[PER], T (&qy)[PER]) {
+  if constexpr (sizeof(T) == 8) {
+#pragma unroll
+    for (int u = 0; u < PER; ++u) qx[u] = ax(u) / dx, qy[u] = ay(u) / dx;
+  } else {
+    unsigned worst = rdx == T(0) ? ~0u : 0u;
+    auto q = [&](T a) -> T {
+      const T q0 = a * rdx;
+      const T r = fma(-q0, dx, a);
+      worst = max(worst, (unsigned)(__builtin_amdgcn_frexp_expf(a) + 99));
+      return copysign(fma(r, rdx, q0), a);
+    };
+#pragma unroll
+    for (int u = 0; u < PER; ++u) qx[u] = q(ax(u)), qy[u] = q(ay(u));
+    if (worst > 200u) {
+      __asm__ volatile("");  // a real branch: keeps the divisions off the common path
+#pragma unroll
+      for (int u = 0; u < PER; ++u) qx[u] = ax(u) / dx, qy[u] = ay(u) / dx;
+    }
+  }
 }
 
 // Tile (tr, tc) for linear index b of the interior rectangle or of the ring.
@@ -54,33 +95,6 @@ __device__ __forceinline__ void tile_linear(bool pml, const TileMap& m, int b, i
     *tc = m.c0 + b % w;
     return;
   }
-  if (b < m.r0 * m.C) {
-    *tr = b / m.C;
-    *tc = b % m.C;
-    return;
-  }
-  b -= m.r0 * m.C;
-  if (b < (m.R - m.r1) * m.C) {
-    *tr = m.r1 + b / m.C;
-    *tc = b % m.C;
-    return;
-  }
-  b -= (m.R - m.r1) * m.C;
-  int per = m.c0 + (m.C - m.c1);
-  *tr = m.r0 + b / per;
-  int k = b % per;
-  *tc = k < m.c0 ? k : m.c1 + (k - m.c0);
-}
-
-// Tile (tr, tc) of this workgroup: interior launches cover the rectangle
-// [r0, r1) x [c0, c1); PML launches enumerate the ring of tiles around it.
-__device__ __forceinline__ void tile_of(bool pml, const TileMap& m, int* tr, int* tc) {
-  if (!pml) {
-    *tr = m.r0 + blockIdx.y;
-    *tc = m.c0 + blockIdx.x;
-    return;
-  }
-  int b = blockIdx.x;
   if (b < m.r0 * m.C) {
     *tr = b / m.C;
     *tc = b % m.C;
@@ -122,13 +136,16 @@ __device__ __forceinline__ bool taps_touch(const TapSet& taps, int I0, int J0, i
 }
 
 // Write this tile's share of every monitor term after sub-step `s`.
-// FIELD(id, li, lj) returns the LDS value of field `id` at local cell.
-template <typename T, int RX, int RY, typename F>
+// FIELD(id, li, lj) returns the LDS value of field `id` at local cell; terms
+// of fields from D0 up (D, which only the owning thread's registers hold)
+// are left to write_taps_own.
+template <typename T, int RX, int RY, int D0, typename F>
 __device__ void write_taps(const TapSet& taps, int s, int I0, int J0, int TXo, int TYo, int a0, int b0,
-                           F field, int slot_base = 0) {
+                           F field, int slot_base) {
   const int tid = threadIdx.x;
   for (int q = 0; q < taps.n; ++q) {
     const Tap& t = taps.t[q];
+    if (t.field >= D0) continue;
     T* out = static_cast<T*>(t.out) + (long long)(t.slot0 + slot_base + s) * t.slot_stride;
     if (t.line == 1) {  // row: fixed i = fix, j = lo + e
       if (t.fix < I0 || t.fix >= I0 + TXo) continue;
@@ -164,414 +181,500 @@ __device__ void write_taps(const TapSet& taps, int s, int I0, int J0, int TXo, i
   }
 }
 
+// The terms of one D field (id `field`): an owned cell (i, j) with value v
+// writes itself (D terms are never averaged; build_taps sees to it).
+template <typename T>
+__device__ __forceinline__ void write_taps_own(const TapSet& taps, int s, int field, int i, int j, T v,
+                                               int slot_base) {
+  for (int q = 0; q < taps.n; ++q) {
+    const Tap& t = taps.t[q];
+    if (t.field != field) continue;
+    T* out = static_cast<T*>(t.out) + (long long)(t.slot0 + slot_base + s) * t.slot_stride;
+    if (t.line == 1) {
+      if (i == t.fix && j >= t.lo && j < t.lo + t.n) out[j - t.lo] = v;
+    } else if (t.line == 2) {
+      if (j == t.fix && i >= t.lo && i < t.lo + t.n) out[i - t.lo] = v;
+    } else if (t.line == 3) {
+      if (i < t.n0 && j < t.n1) out[(long long)i * t.n1 + j] = v;
+    } else if (t.line == 4) {
+      if (i == t.fix && j == t.lo) out[0] = v;
+    }
+  }
+}
+
+__device__ __forceinline__ bool taps_have(const TapSet& taps, int field0) {
+  for (int q = 0; q < taps.n; ++q)
+    if (taps.t[q].field >= field0) return true;
+  return false;
+}
+
+// Does box s reach the region [a0, a0 + RX) x [b0, b0 + RY)?
+__device__ __forceinline__ bool box_touches(const mt_source2d& s, int a0, int b0, int RX, int RY) {
+  return s.present && s.i0 < a0 + RX && s.i1 > a0 && s.j0 < b0 + RY && s.j1 > b0;
+}
+__device__ __forceinline__ bool box_has(const mt_source2d& s, int i, int j) {
+  return i >= s.i0 && i < s.i1 && j >= s.j0 && j < s.j1;
+}
+template <typename T>
+__device__ __forceinline__ T box_w(const mt_source2d& s, int i, int j) {
+  return static_cast<const T*>(s.w)[(long long)(i - s.i0) * (s.j1 - s.j0) + (j - s.j0)];
+}
+
+// Row profiles of the region in LDS: (b, a) of the two x-axis profiles, for
+// rows inside the shells (other entries are never read).
+template <typename T, int RX>
+__device__ __forceinline__ void load_rows(const Pml<T>& h, const Pml<T>& e, int a0, int nh, int ne, T* prof) {
+  for (int li = threadIdx.x; li < RX; li += blockDim.x) {
+    const int i = a0 + li;
+    if (i >= 0 && i < nh && h.in(i)) {
+      prof[li] = h.b[i];
+      prof[RX + li] = h.a[i];
+    }
+    if (i >= 1 && i - 1 < ne && e.in(i - 1)) {
+      prof[2 * RX + li] = e.b[i - 1];
+      prof[3 * RX + li] = e.a[i - 1];
+    }
+  }
+}
+
 // ------------------------------------------------------------------- TE
-template <typename T, int TX, int TY, int NS, bool PML>
-__global__ __launch_bounds__(te_block(PML)) void te_tiled(TeTiled<T> p, TapSet taps, int nsub, int write_e) {
-  constexpr int BLK_TE = te_block(PML);
-  constexpr int RX = TX + 2 * NS + 1, RY = TY + 2 * NS + 1, RC = RX * RY;
-  constexpr int PER = (RC + BLK_TE - 1) / BLK_TE;
-  __shared__ T sHz[RC], sDx[RC], sDy[RC], sEx[RC], sEy[RC];
-  // The psi recursions are pointwise (a cell's psi feeds only that cell's
-  // update), so the thread that updates a cell keeps its four psi values in
-  // registers and writes back those of its owned cells at the end.
+template <typename T, int TX, int TY, int NS, int MAXB, bool PML>
+__device__ __forceinline__ void te_tile(const TeTiled<T>& p, const TapSet& taps, int nsub, int write_e, int tr,
+                                        int tc, T* sm) {
+  using S = Shape<TX, TY, NS, MAXB>;
+  constexpr int RX = S::RX, RY = S::RY, RC = S::RC, ROWS = S::ROWS, STR = S::STR, PER = S::PER;
+  T *sHz = sm, *sEx = sm + RC, *sEy = sm + 2 * RC, *prof = sm + 3 * RC;
   constexpr int PP = PML ? PER : 1;
   T vPzy[PP], vPzx[PP], vPyx[PP], vPxy[PP];  // psi_Hzy (Dx, y shell, (i, j-1)), psi_Hzx (Dy, x shell,
                                              // (i-1, j)), psi_Eyx / psi_Exy (Hz, x / y shell, (i, j))
+  T vHz[PER], vDx[PER], vDy[PER], vKx[PER], vKy[PER], vEx[PER], vEy[PER];
   const int nx = p.nx, ny = p.ny;
-  int tr, tc;
-  tile_of(PML, p.map, &tr, &tc);
   const int I0 = tr * TX, J0 = tc * TY;
   const int a0 = I0 - NS - 1, b0 = J0 - NS - 1;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, l0 = tid / RY, lj = tid - l0 * RY;
+  const int i0 = a0 + l0, j = b0 + lj;
   const T dt = p.dt, dx = p.dx, rdx = p.rdx;
-  // A thread updates the same PER cells of the LDS region in every
-  // sub-step, so eps and the D fields of those cells live in its registers:
-  // the update reads them without LDS traffic, and the LDS holds only what
-  // neighbours, taps and the write-back read (fewer bytes per workgroup,
-  // more workgroups per CU).
-  T vDx[PER], vDy[PER], vKx[PER], vKy[PER];
-  {
-    T vHz[PER];
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      int c = tid + u * BLK_TE;
-      int i = a0 + c / RY, j = b0 + c % RY;
-      bool in = c < RC;
-      bool hz = in && i >= 0 && i < nx - 1 && j >= 0 && j < ny - 1;
-      bool ex = in && i >= 0 && i < nx - 1 && j >= 0 && j < ny;
-      bool ey = in && i >= 0 && i < nx && j >= 0 && j < ny - 1;
-      vHz[u] = dget(p.Hz, (long long)i * (ny - 1) + j, hz);
-      vDx[u] = dget(p.Dx, (long long)i * ny + j, ex);
-      vDy[u] = dget(p.Dy, (long long)i * (ny - 1) + j, ey);
-      vKx[u] = ex ? p.eps_x[(long long)i * ny + j] : T(1);
-      vKy[u] = ey ? p.eps_y[(long long)i * (ny - 1) + j] : T(1);
-    }
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      int c = tid + u * BLK_TE;
-      if (c < RC) {
-        sHz[c] = vHz[u];
-        sDx[c] = vDx[u];
-        sDy[c] = vDy[u];
-      }
-    }
-  }
+  auto ok = [&](int u) { return tid < STR && (u < PER - 1 || l0 + u * ROWS < RX); };
+  const bool jhz = j >= 0 && j < ny - 1, jex = j >= 0 && j < ny;   // columns of Hz / Ey and of Ex
+  const bool jin = j >= 1 && j < ny - 1;
+  const bool in_hy = PML && jhz && p.hy.in(j), in_ey = PML && jin && p.ey.in(j - 1);
+  T bhy = T(0), ahy = T(0), bey = T(0), aey = T(0);
   if constexpr (PML) {
+    if (in_hy) bhy = p.hy.b[j], ahy = p.hy.a[j];
+    if (in_ey) bey = p.ey.b[j - 1], aey = p.ey.a[j - 1];
+    load_rows<T, RX>(p.hx, p.ex, a0, nx - 1, nx - 2, prof);
+  }
 #pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      int c = tid + u * BLK_TE;
-      int i = a0 + c / RY, j = b0 + c % RY;
-      bool in = c < RC;
-      bool hz = in && i >= 0 && i < nx - 1 && j >= 0 && j < ny - 1;
-      bool ex = in && i >= 0 && i < nx - 1 && j >= 0 && j < ny;
-      bool ey = in && i >= 0 && i < nx && j >= 0 && j < ny - 1;
-      vPzy[u] = dget(p.pHzy, (long long)i * (ny - 2) + (j - 1), ex && j >= 1 && j < ny - 1 && p.ey.in(j - 1));
+  for (int u = 0; u < PER; ++u) {
+    const int i = i0 + u * ROWS;
+    const bool rx = !PML || (i >= 0 && i < nx - 1), ry = !PML || (i >= 0 && i < nx);
+    const bool hz = ok(u) && rx && (!PML || jhz), ex = ok(u) && rx && (!PML || jex);
+    const bool ey = ok(u) && ry && (!PML || jhz);
+    vHz[u] = dget(p.Hz, (long long)i * (ny - 1) + j, hz);
+    vDx[u] = dget(p.Dx, (long long)i * ny + j, ex);
+    vDy[u] = dget(p.Dy, (long long)i * (ny - 1) + j, ey);
+    vKx[u] = ex ? p.eps_x[(long long)i * ny + j] : T(1);
+    vKy[u] = ey ? p.eps_y[(long long)i * (ny - 1) + j] : T(1);
+    if constexpr (PML) {
+      vPzy[u] = dget(p.pHzy, (long long)i * (ny - 2) + (j - 1), ex && in_ey);
       vPzx[u] = dget(p.pHzx, (long long)(i - 1) * (ny - 1) + j, ey && i >= 1 && i < nx - 1 && p.ex.in(i - 1));
       vPyx[u] = dget(p.pEyx, (long long)i * (ny - 1) + j, hz && p.hx.in(i));
-      vPxy[u] = dget(p.pExy, (long long)i * (ny - 1) + j, hz && p.hy.in(j));
+      vPxy[u] = dget(p.pExy, (long long)i * (ny - 1) + j, hz && in_hy);
     }
   }
+#pragma unroll
+  for (int u = 0; u < PER; ++u)
+    if (ok(u)) sHz[tid + u * STR] = vHz[u];
   __syncthreads();
   // uniform per tile: does the source reach the LDS region, do taps reach the owned block
-  const bool src_tile = p.src.present && p.src.i0 < a0 + RX && p.src.i1 > a0 && p.src.j0 < b0 + RY &&
-                        p.src.j1 > b0;
+  const bool src_tile = box_touches(p.src, a0, b0, RX, RY);
   const bool tap_tile = taps.n && taps_touch(taps, I0, J0, TX, TY);
+  const bool tap_d = tap_tile && taps_have(taps, 3);
+  const bool jown = lj > NS && lj <= NS + TY && tid < STR;
+  auto own = [&](int u) { return jown && l0 + u * ROWS > NS && l0 + u * ROWS <= NS + TX; };
   for (int s = 0; s < nsub; ++s) {
     const T coef = p.coef[s];
     // D half (stepper_te.py:80-103,131-134,160-168)
-    int li = tid / RY, lj = tid % RY;
+    {
+      T qx[PER], qy[PER];
+      auto ax = [&](int u) -> T {
+        const int c = tid + u * STR, i = i0 + u * ROWS;
+        const bool l = ok(u) && lj >= 1 && (!PML || (jin && i >= 0 && i < nx - 1));
+        return l ? vHz[u] - sHz[c - 1] : T(0);
+      };
+      auto ay = [&](int u) -> T {
+        const int c = tid + u * STR, i = i0 + u * ROWS;
+        const bool l = ok(u) && (u > 0 || l0 >= 1) && (!PML || (jhz && i >= 1 && i < nx - 1));
+        return l ? vHz[u] - sHz[c - RY] : T(0);
+      };
+      step_quots<T, PER>(dx, rdx, ax, ay, qx, qy);
 #pragma unroll
-    for (int u = 0; u < PER; ++u, li += BLK_TE / RY, lj += BLK_TE % RY) {
-      if (lj >= RY) {
-        lj -= RY;
-        ++li;
-      }
-      int c = li * RY + lj;
-      if (c >= RC) break;
-      int i = a0 + li, j = b0 + lj;
-      if (!PML || (i >= 0 && i < nx - 1 && j >= 0 && j < ny)) {
-        T dxv = vDx[u];
-        if ((!PML || (j >= 1 && j < ny - 1)) && lj >= 1) {
-          T d = div_c(sHz[c] - sHz[c - 1], dx, rdx);
-          T curl = d;
-          if (PML && p.ey.in(j - 1)) {
-            T ps = p.ey.b[j - 1] * vPzy[PML ? u : 0] + p.ey.a[j - 1] * d;
-            vPzy[PML ? u : 0] = ps;
-            curl = d + ps;
+      for (int u = 0; u < PER; ++u) {
+        const int c = tid + u * STR, i = i0 + u * ROWS, li = l0 + u * ROWS;
+        if (!ok(u)) break;
+        T cx = qx[u], cy = qy[u];
+        if constexpr (PML) {
+          if (in_ey && lj >= 1 && i >= 0 && i < nx - 1) {
+            const T ps = bey * vPzy[u] + aey * cx;
+            vPzy[u] = ps;
+            cx = cx + ps;
           }
-          dxv = dxv + dt * curl;
-        }
-        vDx[u] = dxv;
-        sDx[c] = dxv;
-        sEx[c] = dxv / vKx[u];
-      }
-      if (!PML || (i >= 0 && i < nx && j >= 0 && j < ny - 1)) {
-        T dyv = vDy[u];
-        if ((!PML || (i >= 1 && i < nx - 1)) && li >= 1) {
-          T d = div_c(sHz[c] - sHz[c - RY], dx, rdx);
-          T curl = d;
-          if (PML && p.ex.in(i - 1)) {
-            T ps = p.ex.b[i - 1] * vPzx[PML ? u : 0] + p.ex.a[i - 1] * d;
-            vPzx[PML ? u : 0] = ps;
-            curl = d + ps;
+          if (jhz && (u > 0 || l0 >= 1) && i >= 1 && i < nx - 1 && p.ex.in(i - 1)) {
+            const T ps = prof[2 * RX + li] * vPzx[u] + prof[3 * RX + li] * cy;
+            vPzx[u] = ps;
+            cy = cy + ps;
           }
-          dyv = dyv - dt * curl;
         }
-        if (src_tile && i >= p.src.i0 && i < p.src.i1 && j >= p.src.j0 && j < p.src.j1)
-          dyv = dyv - coef * static_cast<const T*>(p.src.w)[(long long)s * p.src.wstep + (long long)(i - p.src.i0) * (p.src.j1 - p.src.j0) +
+        T dyv = vDy[u] - dt * cy;
+        vDx[u] = vDx[u] + dt * cx;
+        if (src_tile && box_has(p.src, i, j))
+          dyv = dyv - coef * static_cast<const T*>(p.src.w)[(long long)s * p.src.wstep +
+                                                             (long long)(i - p.src.i0) * (p.src.j1 - p.src.j0) +
                                                              (j - p.src.j0)];
         vDy[u] = dyv;
-        sDy[c] = dyv;
-        sEy[c] = dyv / vKy[u];
+        vEx[u] = vDx[u] / vKx[u];
+        vEy[u] = dyv / vKy[u];
+        sEx[c] = vEx[u];
+        sEy[c] = vEy[u];
       }
     }
     __syncthreads();
     // B half (stepper_te.py:106-117)
-    li = tid / RY;
-    lj = tid % RY;
+    {
+      T qx[PER], qy[PER];
+      auto hz = [&](int u) {
+        const int i = i0 + u * ROWS;
+        return ok(u) && lj < RY - 1 && (u < PER - 1 || l0 + u * ROWS < RX - 1) &&
+               (!PML || (jhz && i >= 0 && i < nx - 1));
+      };
+      auto ax = [&](int u) -> T { return hz(u) ? sEx[tid + u * STR + 1] - vEx[u] : T(0); };
+      auto ay = [&](int u) -> T { return hz(u) ? sEy[tid + u * STR + RY] - vEy[u] : T(0); };
+      step_quots<T, PER>(dx, rdx, ax, ay, qx, qy);
 #pragma unroll
-    for (int u = 0; u < PER; ++u, li += BLK_TE / RY, lj += BLK_TE % RY) {
-      if (lj >= RY) {
-        lj -= RY;
-        ++li;
-      }
-      int c = li * RY + lj;
-      if (c >= RC) break;
-      int i = a0 + li, j = b0 + lj;
-      if ((!PML || (i >= 0 && i < nx - 1 && j >= 0 && j < ny - 1)) && li < RX - 1 && lj < RY - 1) {
-        T dEy = div_c(sEy[c + RY] - sEy[c], dx, rdx);
-        T dEx = div_c(sEx[c + 1] - sEx[c], dx, rdx);
-        T a1 = dEy;
-        if (PML && p.hx.in(i)) {
-          T ps = p.hx.b[i] * vPyx[PML ? u : 0] + p.hx.a[i] * dEy;
-          vPyx[PML ? u : 0] = ps;
-          a1 = dEy + ps;
+      for (int u = 0; u < PER; ++u) {
+        const int c = tid + u * STR, i = i0 + u * ROWS, li = l0 + u * ROWS;
+        if (!ok(u)) break;
+        T a1 = qy[u];
+        if constexpr (PML) {
+          const bool h = lj < RY - 1 && li < RX - 1 && jhz && i >= 0 && i < nx - 1;
+          if (h && p.hx.in(i)) {
+            const T ps = prof[li] * vPyx[u] + prof[RX + li] * qy[u];
+            vPyx[u] = ps;
+            a1 = a1 + ps;
+          }
+          a1 = a1 - qx[u];
+          if (h && in_hy) {
+            const T ps = bhy * vPxy[u] + ahy * qx[u];
+            vPxy[u] = ps;
+            a1 = a1 - ps;
+          }
+        } else {
+          a1 = a1 - qx[u];
         }
-        T curl = a1 - dEx;
-        if (PML && p.hy.in(j)) {
-          T ps = p.hy.b[j] * vPxy[PML ? u : 0] + p.hy.a[j] * dEx;
-          vPxy[PML ? u : 0] = ps;
-          curl = curl - ps;
-        }
-        sHz[c] = sHz[c] - dt * curl;
+        vHz[u] = vHz[u] - dt * a1;
+        sHz[c] = vHz[u];
       }
     }
     __syncthreads();
     if (tap_tile) {
-      write_taps<T, RX, RY>(taps, s, I0, J0, TX, TY, a0, b0, [&](int f, int li, int lj) -> T {
-        int c = li * RY + lj;
-        return f == 0 ? sHz[c] : f == 1 ? sEx[c] : f == 2 ? sEy[c] : f == 3 ? sDx[c] : sDy[c];
-      });
+      write_taps<T, RX, RY, 3>(
+          taps, s, I0, J0, TX, TY, a0, b0,
+          [&](int f, int li, int lj) -> T {
+            int c = li * RY + lj;
+            return f == 0 ? sHz[c] : f == 1 ? sEx[c] : sEy[c];
+          },
+          0);
+      if (tap_d) {
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+          const int i = i0 + u * ROWS;
+          if (!own(u)) continue;
+          if (i < nx - 1 && j < ny) write_taps_own<T>(taps, s, 3, i, j, vDx[u], 0);
+          if (i < nx && j < ny - 1) write_taps_own<T>(taps, s, 4, i, j, vDy[u], 0);
+        }
+      }
       __syncthreads();
     }
   }
-  // write back the owned block
-  for (int c = tid; c < TX * TY; c += BLK_TE) {
-    int i = I0 + c / TY, j = J0 + c % TY;
-    int lc = (i - a0) * RY + (j - b0);
+  // write back the owned cells from the registers of the threads that updated them
+#pragma unroll
+  for (int u = 0; u < PER; ++u) {
+    const int i = i0 + u * ROWS;
+    if (!own(u)) continue;
+    const long long h = (long long)i * (ny - 1) + j, e = (long long)i * ny + j;
     if (i < nx - 1 && j < ny - 1) {
-      long long h = (long long)i * (ny - 1) + j;
-      p.oHz[h] = sHz[lc];
+      p.oHz[h] = vHz[u];
+      if constexpr (PML) {
+        if (p.hx.in(i)) p.oEyx[h] = vPyx[u];
+        if (in_hy) p.oExy[h] = vPxy[u];
+      }
     }
     if (i < nx - 1 && j < ny) {
-      long long h = (long long)i * ny + j;
-      p.oDx[h] = sDx[lc];
-      if (write_e) p.Ex[h] = sEx[lc];
+      p.oDx[e] = vDx[u];
+      if (write_e) p.Ex[e] = vEx[u];
+      if constexpr (PML)
+        if (in_ey) p.oHzy[(long long)i * (ny - 2) + (j - 1)] = vPzy[u];
     }
     if (i < nx && j < ny - 1) {
-      long long h = (long long)i * (ny - 1) + j;
-      p.oDy[h] = sDy[lc];
-      if (write_e) p.Ey[h] = sEy[lc];
-    }
-  }
-  if constexpr (PML) {  // psi of the owned cells, from the registers of the threads that updated them
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      int c = tid + u * BLK_TE;
-      int i = a0 + c / RY, j = b0 + c % RY;
-      if (c >= RC || i < I0 || i >= I0 + TX || j < J0 || j >= J0 + TY) continue;
-      if (i < nx - 1 && j < ny - 1) {
-        long long h = (long long)i * (ny - 1) + j;
-        if (p.hx.in(i)) p.oEyx[h] = vPyx[u];
-        if (p.hy.in(j)) p.oExy[h] = vPxy[u];
-      }
-      if (i < nx - 1 && j < ny && j >= 1 && j < ny - 1 && p.ey.in(j - 1))
-        p.oHzy[(long long)i * (ny - 2) + (j - 1)] = vPzy[u];
-      if (i < nx && j < ny - 1 && i >= 1 && i < nx - 1 && p.ex.in(i - 1))
-        p.oHzx[(long long)(i - 1) * (ny - 1) + j] = vPzx[u];
+      p.oDy[h] = vDy[u];
+      if (write_e) p.Ey[h] = vEy[u];
+      if constexpr (PML)
+        if (i >= 1 && i < nx - 1 && p.ex.in(i - 1)) p.oHzx[(long long)(i - 1) * (ny - 1) + j] = vPzx[u];
     }
   }
 }
 
 // ------------------------------------------------------------------- TM
-template <typename T, int TX, int TY, int NS, bool PML>
+template <typename T, int TX, int TY, int NS, int MAXB, bool PML>
 __device__ __forceinline__ void tm_tile(const TmTiled<T>& p, const TapSet& taps, int nsub, int tape_s0, int tr,
-                                        int tc, int slot_base, int coef_t0) {
-  constexpr int RX = TX + 2 * NS + 1, RY = TY + 2 * NS + 1, RC = RX * RY;
-  constexpr int PER = (RC + BLK_TM - 1) / BLK_TM;
-  __shared__ T sEz[RC], sDz[RC], sHx[RC], sHy[RC];
-  // psi in the registers of the thread that updates the cell (as in te_tiled)
+                                        int tc, int slot_base, int coef_t0, T* sm) {
+  using S = Shape<TX, TY, NS, MAXB>;
+  constexpr int RX = S::RX, RY = S::RY, RC = S::RC, ROWS = S::ROWS, STR = S::STR, PER = S::PER;
+  T *sEz = sm, *sHx = sm + RC, *sHy = sm + 2 * RC, *prof = sm + 3 * RC;
   constexpr int PP = PML ? PER : 1;
   T vPzy[PP], vPzx[PP], vPyx[PP], vPxy[PP];  // psi_Ezy (Hx, y shell, (i, j)), psi_Ezx (Hy, x shell, (i, j)),
                                              // psi_Hyx / psi_Hxy (Dz, x / y shell, (i-1, jj))
+  T vEz[PER], vDz[PER], vHx[PER], vHy[PER], vK[PER];
   const int nx = p.nx, ny = p.ny, ny_e = p.ny_e;
   const int I0 = tr * TX, J0 = tc * TY;
   const int a0 = I0 - NS - 1, b0 = J0 - NS - 1;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, l0 = tid / RY, lj = tid - l0 * RY;
+  const int i0 = a0 + l0, j = b0 + lj, jj = j - (p.y_pmc ? 0 : 1);
   const T dt = p.dt, dx = p.dx, rdx = p.rdx;
-  const int joff = p.y_pmc ? 0 : 1;
-  // eps and Dz of the PER cells this thread updates stay in its registers
-  // across sub-steps (as in te_tiled)
-  T vDz[PER], vK[PER];
-  {
-    T vEz[PER], vHx[PER], vHy[PER];
+  auto ok = [&](int u) { return tid < STR && (u < PER - 1 || l0 + u * ROWS < RX); };
+  const bool jez = j >= 0 && j < ny, jhx = j >= 0 && j < ny - 1;
+  const bool jlive = jez && jj >= 0 && jj < ny_e;   // columns the D half updates
+  const bool in_hy = PML && jhx && p.hy.in(j), in_ey = PML && jlive && p.ey.in(jj);
+  T bhy = T(0), ahy = T(0), bey = T(0), aey = T(0);
+  if constexpr (PML) {
+    if (in_hy) bhy = p.hy.b[j], ahy = p.hy.a[j];
+    if (in_ey) bey = p.ey.b[jj], aey = p.ey.a[jj];
+    load_rows<T, RX>(p.hx, p.ex, a0, nx - 1, nx - 2, prof);
+  }
 #pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      int c = tid + u * BLK_TM;
-      int i = a0 + c / RY, j = b0 + c % RY;
-      bool ez = c < RC && i >= 0 && i < nx && j >= 0 && j < ny;
-      vEz[u] = dget(p.Ez, (long long)i * ny + j, ez);
-      vDz[u] = dget(p.Dz, (long long)i * ny + j, ez);
-      vHx[u] = dget(p.Hx, (long long)i * (ny - 1) + j, ez && j < ny - 1);
-      vHy[u] = dget(p.Hy, (long long)i * ny + j, ez && i < nx - 1);
-      vK[u] = ez ? p.eps[(long long)i * ny + j] : T(1);
-    }
-#pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      int c = tid + u * BLK_TM;
-      if (c < RC) {
-        sEz[c] = vEz[u];
-        sDz[c] = vDz[u];
-        sHx[c] = vHx[u];
-        sHy[c] = vHy[u];
-      }
+  for (int u = 0; u < PER; ++u) {
+    const int i = i0 + u * ROWS;
+    const bool ez = ok(u) && (!PML || (i >= 0 && i < nx && jez));
+    const bool hx = ez && (!PML || jhx), hy = ez && (!PML || i < nx - 1);
+    const long long e = (long long)i * ny + j;
+    vEz[u] = dget(p.Ez, e, ez);
+    vHx[u] = dget(p.Hx, (long long)i * (ny - 1) + j, hx);
+    vHy[u] = dget(p.Hy, e, hy);
+    vDz[u] = dget(p.Dz, e, ez);
+    vK[u] = ez ? p.eps[e] : T(1);
+    if constexpr (PML) {
+      const bool live = ez && i >= 1 && i < nx - 1 && jlive;
+      const long long q = (long long)(i - 1) * ny_e + jj;
+      vPzy[u] = dget(p.pEzy, (long long)i * (ny - 1) + j, hx && in_hy);
+      vPzx[u] = dget(p.pEzx, e, hy && p.hx.in(i));
+      vPyx[u] = dget(p.pHyx, q, live && p.ex.in(i - 1));
+      vPxy[u] = dget(p.pHxy, q, live && in_ey);
     }
   }
-  if constexpr (PML) {
 #pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      int c = tid + u * BLK_TM;
-      int i = a0 + c / RY, j = b0 + c % RY;
-      bool ez = c < RC && i >= 0 && i < nx && j >= 0 && j < ny;
-      bool hx = ez && j < ny - 1;
-      bool hy = ez && i < nx - 1;
-      vPzy[u] = dget(p.pEzy, (long long)i * (ny - 1) + j, hx && p.hy.in(j));
-      vPzx[u] = dget(p.pEzx, (long long)i * ny + j, hy && p.hx.in(i));
-      int jj = j - joff;
-      bool live = ez && i >= 1 && i < nx - 1 && jj >= 0 && jj < ny_e;
-      long long q = (long long)(i - 1) * ny_e + jj;
-      vPyx[u] = dget(p.pHyx, q, live && p.ex.in(i - 1));
-      vPxy[u] = dget(p.pHxy, q, live && p.ey.in(jj));
+  for (int u = 0; u < PER; ++u) {
+    const int c = tid + u * STR;
+    if (ok(u)) {
+      sEz[c] = vEz[u];
+      sHx[c] = vHx[u];
+      sHy[c] = vHy[u];
     }
   }
   __syncthreads();
-  // uniform per tile: does the source reach the LDS region, do taps reach the owned block
-  const bool src_tile = p.src.present && p.src.i0 < a0 + RX && p.src.i1 > a0 && p.src.j0 < b0 + RY &&
-                        p.src.j1 > b0;
-  const bool hx_tile = p.hsrc[0].present && p.hsrc[0].i0 < a0 + RX && p.hsrc[0].i1 > a0 &&
-                       p.hsrc[0].j0 < b0 + RY && p.hsrc[0].j1 > b0;
-  const bool hy_tile = p.hsrc[1].present && p.hsrc[1].i0 < a0 + RX && p.hsrc[1].i1 > a0 &&
-                       p.hsrc[1].j0 < b0 + RY && p.hsrc[1].j1 > b0;
+  // uniform per tile: do the sources reach the LDS region, do taps reach the owned block
+  const bool src_tile = box_touches(p.src, a0, b0, RX, RY);
+  const bool hx_tile = box_touches(p.hsrc[0], a0, b0, RX, RY), hy_tile = box_touches(p.hsrc[1], a0, b0, RX, RY);
   const bool tap_tile = taps.n && taps_touch(taps, I0, J0, TX, TY);
+  const bool tap_d = tap_tile && taps_have(taps, 3);
+  const bool jown = lj > NS && lj <= NS + TY && tid < STR && j < ny;
+  auto own = [&](int u) {
+    return jown && l0 + u * ROWS > NS && l0 + u * ROWS <= NS + TX && i0 + u * ROWS < nx;
+  };
   for (int s = 0; s < nsub; ++s) {
     const T coef = p.coef_tab ? p.coef_tab[coef_t0 + s] : p.coef[s];
     const T hc = p.hcoef_tab ? p.hcoef_tab[coef_t0 + s] : p.hcoef[s];
     // B half (stepper_tm.py:85-92,126-128)
-    int li = tid / RY, lj = tid % RY;
+    {
+      T qx[PER], qy[PER];
+      auto ay = [&](int u) -> T {
+        const int i = i0 + u * ROWS;
+        const bool l = ok(u) && lj < RY - 1 && (!PML || (i >= 0 && i < nx && jhx));
+        return l ? sEz[tid + u * STR + 1] - vEz[u] : T(0);
+      };
+      auto ax = [&](int u) -> T {
+        const int i = i0 + u * ROWS;
+        const bool l = ok(u) && (u < PER - 1 || l0 + u * ROWS < RX - 1) &&
+                       (!PML || (i >= 0 && i < nx - 1 && jez));
+        return l ? sEz[tid + u * STR + RY] - vEz[u] : T(0);
+      };
+      step_quots<T, PER>(dx, rdx, ax, ay, qx, qy);
 #pragma unroll
-    for (int u = 0; u < PER; ++u, li += BLK_TM / RY, lj += BLK_TM % RY) {
-      if (lj >= RY) {
-        lj -= RY;
-        ++li;
-      }
-      int c = li * RY + lj;
-      if (c >= RC) break;
-      int i = a0 + li, j = b0 + lj;
-      if (PML && (i < 0 || i >= nx || j < 0 || j >= ny)) continue;
-      T ez = sEz[c];
-      if ((!PML || j < ny - 1) && lj < RY - 1) {
-        T d = div_c(sEz[c + 1] - ez, dx, rdx);
-        T curl = d;
-        if (PML && p.hy.in(j)) {
-          T ps = p.hy.b[j] * vPzy[PML ? u : 0] + p.hy.a[j] * d;
-          vPzy[PML ? u : 0] = ps;
-          curl = d + ps;
+      for (int u = 0; u < PER; ++u) {
+        const int c = tid + u * STR, i = i0 + u * ROWS, li = l0 + u * ROWS;
+        if (!ok(u)) break;
+        T cy = qy[u], cx = qx[u];
+        if constexpr (PML) {
+          if (in_hy && lj < RY - 1 && i >= 0 && i < nx) {
+            const T ps = bhy * vPzy[u] + ahy * cy;
+            vPzy[u] = ps;
+            cy = cy + ps;
+          }
+          if (jez && li < RX - 1 && i >= 0 && i < nx - 1 && p.hx.in(i)) {
+            const T ps = prof[li] * vPzx[u] + prof[RX + li] * cx;
+            vPzx[u] = ps;
+            cx = cx + ps;
+          }
         }
-        T hxv = sHx[c] - dt * curl;
-        if (hx_tile && i >= p.hsrc[0].i0 && i < p.hsrc[0].i1 && j >= p.hsrc[0].j0 && j < p.hsrc[0].j1)
-          hxv = hxv - hc * static_cast<const T*>(p.hsrc[0].w)[(long long)(i - p.hsrc[0].i0) *
-                                                                   (p.hsrc[0].j1 - p.hsrc[0].j0) +
-                                                               (j - p.hsrc[0].j0)];  // stepper_tm.py:190-191
+        T hxv = vHx[u] - dt * cy, hyv = vHy[u] + dt * cx;
+        if (hx_tile && box_has(p.hsrc[0], i, j)) hxv = hxv - hc * box_w<T>(p.hsrc[0], i, j);  // stepper_tm.py:190-191
+        if (hy_tile && box_has(p.hsrc[1], i, j)) hyv = hyv - hc * box_w<T>(p.hsrc[1], i, j);  // stepper_tm.py:188-189
+        vHx[u] = hxv;
+        vHy[u] = hyv;
         sHx[c] = hxv;
-      }
-      if ((!PML || i < nx - 1) && li < RX - 1) {
-        T d = div_c(sEz[c + RY] - ez, dx, rdx);
-        T curl = d;
-        if (PML && p.hx.in(i)) {
-          T ps = p.hx.b[i] * vPzx[PML ? u : 0] + p.hx.a[i] * d;
-          vPzx[PML ? u : 0] = ps;
-          curl = d + ps;
-        }
-        T hyv = sHy[c] + dt * curl;
-        if (hy_tile && i >= p.hsrc[1].i0 && i < p.hsrc[1].i1 && j >= p.hsrc[1].j0 && j < p.hsrc[1].j1)
-          hyv = hyv - hc * static_cast<const T*>(p.hsrc[1].w)[(long long)(i - p.hsrc[1].i0) *
-                                                                   (p.hsrc[1].j1 - p.hsrc[1].j0) +
-                                                               (j - p.hsrc[1].j0)];  // stepper_tm.py:188-189
         sHy[c] = hyv;
       }
     }
     __syncthreads();
-    // D half (stepper_tm.py:130-166,197-200,226-227)
-    li = tid / RY;
-    lj = tid % RY;
+    // D half (stepper_tm.py:130-166,197-200,226-227).  Under y_pmc the H
+    // beyond a wall is zero: those LDS cells were loaded as zero and no B
+    // half updates them.
+    {
+      T qx[PER], qy[PER];
+      auto lv = [&](int u) {
+        const int i = i0 + u * ROWS;
+        return ok(u) && lj >= 1 && (u > 0 || l0 >= 1) && (!PML || (jlive && i >= 1 && i < nx - 1));
+      };
+      auto ax = [&](int u) -> T { return lv(u) ? vHx[u] - sHx[tid + u * STR - 1] : T(0); };
+      auto ay = [&](int u) -> T { return lv(u) ? vHy[u] - sHy[tid + u * STR - RY] : T(0); };
+      step_quots<T, PER>(dx, rdx, ax, ay, qx, qy);
 #pragma unroll
-    for (int u = 0; u < PER; ++u, li += BLK_TM / RY, lj += BLK_TM % RY) {
-      if (lj >= RY) {
-        lj -= RY;
-        ++li;
-      }
-      int c = li * RY + lj;
-      if (c >= RC) break;
-      int i = a0 + li, j = b0 + lj;
-      if (PML && (i < 0 || i >= nx || j < 0 || j >= ny)) continue;
-      T dz = vDz[u];
-      bool live = !PML || (i >= 1 && i < nx - 1 && (p.y_pmc || (j >= 1 && j < ny - 1)));
-      if (live && li >= 1 && lj >= 1) {
-        T hx1 = (!PML || j < ny - 1) ? sHx[c] : T(0);
-        T hx0 = (!PML || j >= 1) ? sHx[c - 1] : T(0);
-        T dHx = div_c(hx1 - hx0, dx, rdx);
-        T dHy = div_c(sHy[c] - sHy[c - RY], dx, rdx);
-        int ii = i - 1, jj = j - joff;
-        T a1 = dHy;
-        if (PML && p.ex.in(ii)) {
-          T ps = p.ex.b[ii] * vPyx[PML ? u : 0] + p.ex.a[ii] * dHy;
-          vPyx[PML ? u : 0] = ps;
-          a1 = dHy + ps;
+      for (int u = 0; u < PER; ++u) {
+        const int c = tid + u * STR, i = i0 + u * ROWS, li = l0 + u * ROWS;
+        if (!ok(u)) break;
+        T curl = qy[u];
+        if constexpr (PML) {
+          const bool live = lj >= 1 && (u > 0 || l0 >= 1) && jlive && i >= 1 && i < nx - 1;
+          if (live && p.ex.in(i - 1)) {
+            const T ps = prof[2 * RX + li] * vPyx[u] + prof[3 * RX + li] * qy[u];
+            vPyx[u] = ps;
+            curl = curl + ps;
+          }
+          curl = curl - qx[u];
+          if (live && in_ey) {
+            const T ps = bey * vPxy[u] + aey * qx[u];
+            vPxy[u] = ps;
+            curl = curl - ps;
+          }
+        } else {
+          curl = curl - qx[u];
         }
-        T curl = a1 - dHx;
-        if (PML && p.ey.in(jj)) {
-          T ps = p.ey.b[jj] * vPxy[PML ? u : 0] + p.ey.a[jj] * dHx;
-          vPxy[PML ? u : 0] = ps;
-          curl = curl - ps;
-        }
-        dz = dz + dt * curl;
+        T dz = vDz[u] + dt * curl;
+        if (src_tile && box_has(p.src, i, j))
+          dz = dz - coef * static_cast<const T*>(p.src.w)[(long long)s * p.src.wstep +
+                                                          (long long)(i - p.src.i0) * (p.src.j1 - p.src.j0) +
+                                                          (j - p.src.j0)];
+        vDz[u] = dz;
+        vEz[u] = dz / vK[u];
+        sEz[c] = vEz[u];
       }
-      if (src_tile && i >= p.src.i0 && i < p.src.i1 && j >= p.src.j0 && j < p.src.j1)
-        dz = dz - coef * static_cast<const T*>(p.src.w)[(long long)s * p.src.wstep + (long long)(i - p.src.i0) * (p.src.j1 - p.src.j0) +
-                                                        (j - p.src.j0)];
-      vDz[u] = dz;
-      sDz[c] = dz;
-      sEz[c] = dz / vK[u];
     }
     __syncthreads();
     if (p.tape) {
-      for (int c = tid; c < TX * TY; c += BLK_TM) {
-        int i = I0 + c / TY, j = J0 + c % TY;
-        if (i < nx && j < ny)
-          p.tape[(long long)(tape_s0 + s) * nx * ny + (long long)i * ny + j] = sEz[(i - a0) * RY + (j - b0)];
-      }
+#pragma unroll
+      for (int u = 0; u < PER; ++u)
+        if (own(u)) p.tape[(long long)(tape_s0 + s) * nx * ny + (long long)(i0 + u * ROWS) * ny + j] = vEz[u];
     }
     if (tap_tile) {
-      write_taps<T, RX, RY>(taps, s, I0, J0, TX, TY, a0, b0, [&](int f, int li, int lj) -> T {
-        int c = li * RY + lj;
-        return f == 0 ? sEz[c] : f == 1 ? sHx[c] : f == 2 ? sHy[c] : sDz[c];
-      }, slot_base);
+      write_taps<T, RX, RY, 3>(
+          taps, s, I0, J0, TX, TY, a0, b0,
+          [&](int f, int li, int lj) -> T {
+            int c = li * RY + lj;
+            return f == 0 ? sEz[c] : f == 1 ? sHx[c] : sHy[c];
+          },
+          slot_base);
+      if (tap_d) {
+#pragma unroll
+        for (int u = 0; u < PER; ++u)
+          if (own(u)) write_taps_own<T>(taps, s, 3, i0 + u * ROWS, j, vDz[u], slot_base);
+      }
       __syncthreads();
     }
   }
-  for (int c = tid; c < TX * TY; c += BLK_TM) {
-    int i = I0 + c / TY, j = J0 + c % TY;
-    if (i >= nx || j >= ny) continue;
-    int lc = (i - a0) * RY + (j - b0);
-    long long e = (long long)i * ny + j;
-    p.oEz[e] = sEz[lc];
-    p.oDz[e] = sDz[lc];
-    if (j < ny - 1) p.oHx[(long long)i * (ny - 1) + j] = sHx[lc];
-    if (i < nx - 1) p.oHy[e] = sHy[lc];
-  }
-  if constexpr (PML) {  // psi of the owned cells, from the registers of the threads that updated them
+  // write back the owned cells from the registers of the threads that updated them
 #pragma unroll
-    for (int u = 0; u < PER; ++u) {
-      int c = tid + u * BLK_TM;
-      int i = a0 + c / RY, j = b0 + c % RY;
-      if (c >= RC || i < I0 || i >= I0 + TX || j < J0 || j >= J0 + TY || i >= nx || j >= ny) continue;
-      if (j < ny - 1 && p.hy.in(j)) p.oEzy[(long long)i * (ny - 1) + j] = vPzy[u];
-      if (i < nx - 1 && p.hx.in(i)) p.oEzx[(long long)i * ny + j] = vPzx[u];
-      int jj = j - joff;
-      if (i >= 1 && i < nx - 1 && jj >= 0 && jj < ny_e) {
-        long long q = (long long)(i - 1) * ny_e + jj;
+  for (int u = 0; u < PER; ++u) {
+    const int i = i0 + u * ROWS;
+    if (!own(u)) continue;
+    const long long e = (long long)i * ny + j;
+    p.oEz[e] = vEz[u];
+    p.oDz[e] = vDz[u];
+    if (j < ny - 1) p.oHx[(long long)i * (ny - 1) + j] = vHx[u];
+    if (i < nx - 1) p.oHy[e] = vHy[u];
+    if constexpr (PML) {
+      if (in_hy) p.oEzy[(long long)i * (ny - 1) + j] = vPzy[u];
+      if (i < nx - 1 && p.hx.in(i)) p.oEzx[e] = vPzx[u];
+      if (i >= 1 && i < nx - 1 && jlive) {
+        const long long q = (long long)(i - 1) * ny_e + jj;
         if (p.ex.in(i - 1)) p.oHyx[q] = vPyx[u];
-        if (p.ey.in(jj)) p.oHxy[q] = vPxy[u];
+        if (in_ey) p.oHxy[q] = vPxy[u];
       }
     }
   }
 }
 
-template <typename T, int TX, int TY, int NS, bool PML>
-__global__ __launch_bounds__(BLK_TM) void tm_tiled(TmTiled<T> p, TapSet taps, int nsub, int tape_s0) {
+// ---------------------------------------------------------------- kernels
+// Threads per workgroup, at most.  TM tiles and CPML tiles take up to 1024
+// (few cells per thread: their launches are latency chains); TE interior
+// tiles of the large shapes take 512 (on 2048^2 that launch is
+// arithmetic-bound and 1024-thread tiles measured slower, 98 -> 123 us).
+constexpr int kMaxTm = 1024;
+template <int TX, int TY, int NS>
+constexpr int te_max(bool pml) {
+  return pml || (TX + 2 * NS + 1) * (TY + 2 * NS + 1) <= 1100 ? 1024 : 512;
+}
+template <typename T, int TX, int TY, int NS, int MAXB, bool PML>
+constexpr int lds_elems() {
+  using S = Shape<TX, TY, NS, MAXB>;
+  return 3 * S::RC + (PML ? 4 * S::RX : 0);
+}
+
+// Which tiles a launch covers: the interior rectangle, the ring around it,
+// or (one launch) all of them, each workgroup taking its tile's path.
+enum { kInterior, kRing, kAll };
+
+template <int MODE>
+__device__ __forceinline__ bool pick_tile(const TileMap& m, int* tr, int* tc) {
+  if constexpr (MODE == kAll) {
+    *tr = blockIdx.x / m.C;
+    *tc = blockIdx.x % m.C;
+    return !(*tr >= m.r0 && *tr < m.r1 && *tc >= m.c0 && *tc < m.c1);
+  }
+  tile_linear(MODE == kRing, m, blockIdx.x, tr, tc);
+  return MODE == kRing;
+}
+
+template <typename T, int TX, int TY, int NS, int MAXB, int MODE>
+__global__ __launch_bounds__((Shape<TX, TY, NS, MAXB>::BLK)) void te_tiled(TeTiled<T> p, TapSet taps, int nsub,
+                                                                          int write_e) {
+  __shared__ T sm[lds_elems<T, TX, TY, NS, MAXB, MODE != kInterior>()];
   int tr, tc;
-  tile_of(PML, p.map, &tr, &tc);
-  tm_tile<T, TX, TY, NS, PML>(p, taps, nsub, tape_s0, tr, tc, 0, 0);
+  const bool pml = pick_tile<MODE>(p.map, &tr, &tc);
+  if (MODE == kRing || (MODE == kAll && pml))
+    te_tile<T, TX, TY, NS, MAXB, true>(p, taps, nsub, write_e, tr, tc, sm);
+  else
+    te_tile<T, TX, TY, NS, MAXB, false>(p, taps, nsub, write_e, tr, tc, sm);
+}
+
+template <typename T, int TX, int TY, int NS, int MODE>
+__global__ __launch_bounds__((Shape<TX, TY, NS, kMaxTm>::BLK)) void tm_tiled(TmTiled<T> p, TapSet taps, int nsub,
+                                                                           int tape_s0) {
+  __shared__ T sm[lds_elems<T, TX, TY, NS, kMaxTm, MODE != kInterior>()];
+  int tr, tc;
+  const bool pml = pick_tile<MODE>(p.map, &tr, &tc);
+  if (MODE == kRing || (MODE == kAll && pml))
+    tm_tile<T, TX, TY, NS, kMaxTm, true>(p, taps, nsub, tape_s0, tr, tc, 0, 0, sm);
+  else
+    tm_tile<T, TX, TY, NS, kMaxTm, false>(p, taps, nsub, tape_s0, tr, tc, 0, 0, sm);
 }
 
 // FP32 interior tiles held to 64 VGPRs (eight waves per SIMD): two
@@ -579,21 +682,26 @@ __global__ __launch_bounds__(BLK_TM) void tm_tiled(TmTiled<T> p, TapSet taps, in
 // other's barrier and load latency.  Ring tiles (CPML psi) and FP64 keep the
 // plain bound.
 template <typename T, int TX, int TY, int NS>
-__global__ __launch_bounds__(BLK_TM) __attribute__((amdgpu_waves_per_eu(8, 8))) void tm_tiled_in2(
-    TmTiled<T> p, TapSet taps, int nsub, int tape_s0) {
+__global__ __launch_bounds__((Shape<TX, TY, NS, kMaxTm>::BLK)) __attribute__((amdgpu_waves_per_eu(8, 8))) void
+tm_tiled_in2(TmTiled<T> p, TapSet taps, int nsub, int tape_s0) {
+  __shared__ T sm[lds_elems<T, TX, TY, NS, kMaxTm, false>()];
   int tr, tc;
-  tile_of(false, p.map, &tr, &tc);
-  tm_tile<T, TX, TY, NS, false>(p, taps, nsub, tape_s0, tr, tc, 0, 0);
+  tile_linear(false, p.map, blockIdx.x, &tr, &tc);
+  tm_tile<T, TX, TY, NS, kMaxTm, false>(p, taps, nsub, tape_s0, tr, tc, 0, 0, sm);
 }
 
 // Persistent batched form: every workgroup walks the flattened (variant,
-// tile) work list of all variants.  Per-variant problems (both ping-pong
-// orientations), taps and tile maps live in device memory, so the launch
-// depends only on scalars and can be captured in a graph and replayed.
-template <typename T, int TX, int TY, int NS, bool PML>
-__device__ __forceinline__ void tm_batch_body(const TmBatchVar<T>* vars, const int* prefix, int nvar, int nsub,
-                                              int parity, int t0, int slot_base, int tape_s0) {
-  const int total = prefix[nvar];
+// tile) work list of all variants: the interior tiles, the ring tiles, or
+// (kAll) the ring tiles and then the interior ones.  Per-variant problems
+// (both ping-pong orientations), taps and tile maps live in device memory, so
+// the launch depends only on scalars and can be captured in a graph and
+// replayed.
+template <typename T, int TX, int TY, int NS, int MODE>
+__device__ __forceinline__ void tm_batch_body(const TmBatchVar<T>* vars, const int* pre_in, const int* pre_ring,
+                                              int nvar, int nsub, int parity, int t0, int slot_base, int tape_s0,
+                                              T* sm) {
+  const int n_ring = MODE == kInterior ? 0 : pre_ring[nvar];
+  const int total = n_ring + (MODE == kRing ? 0 : pre_in[nvar]);
   // XCD-aware order: workgroups are dealt to the eight XCDs round robin, so
   // the blocks of XCD x (blockIdx % 8 == x) share the contiguous item range
   // [x * chunk, (x + 1) * chunk): neighbouring tiles, whose halos overlap,
@@ -601,33 +709,43 @@ __device__ __forceinline__ void tm_batch_body(const TmBatchVar<T>* vars, const i
   const int x = blockIdx.x & 7, nx8 = ((int)gridDim.x - x + 7) >> 3;
   const int chunk = (total + 7) >> 3, end = min(total, (x + 1) * chunk);
   for (int item = x * chunk + (int)(blockIdx.x >> 3); item < end; item += nx8) {
+    const bool ring = MODE == kRing || (MODE == kAll && item < n_ring);
+    const int* prefix = ring ? pre_ring : pre_in;
+    const int it = ring ? item : item - n_ring;
     int lo = 0, hi = nvar;
     while (hi - lo > 1) {
       int mid = (lo + hi) >> 1;
-      if (prefix[mid] <= item) lo = mid;
+      if (prefix[mid] <= it) lo = mid;
       else hi = mid;
     }
     const TmBatchVar<T>& V = vars[lo];
     const TmTiled<T>& p = parity ? V.pB : V.pA;
     int tr, tc;
-    tile_linear(PML, p.map, item - prefix[lo], &tr, &tc);
-    tm_tile<T, TX, TY, NS, PML>(p, V.taps, nsub, tape_s0, tr, tc, slot_base, t0);
+    tile_linear(ring, p.map, it - prefix[lo], &tr, &tc);
+    if (MODE == kRing || (MODE == kAll && ring))
+      tm_tile<T, TX, TY, NS, kMaxTm, true>(p, V.taps, nsub, tape_s0, tr, tc, slot_base, t0, sm);
+    else
+      tm_tile<T, TX, TY, NS, kMaxTm, false>(p, V.taps, nsub, tape_s0, tr, tc, slot_base, t0, sm);
     __syncthreads();
   }
 }
 
-template <typename T, int TX, int TY, int NS, bool PML>
-__global__ __launch_bounds__(BLK_TM) void tm_batch(const TmBatchVar<T>* vars, const int* prefix, int nvar,
-                                                int nsub, int parity, int t0, int slot_base, int tape_s0) {
-  tm_batch_body<T, TX, TY, NS, PML>(vars, prefix, nvar, nsub, parity, t0, slot_base, tape_s0);
+template <typename T, int TX, int TY, int NS, int MODE>
+__global__ __launch_bounds__((Shape<TX, TY, NS, kMaxTm>::BLK)) void tm_batch(const TmBatchVar<T>* vars,
+                                                                           const int* pre_in, const int* pre_ring,
+                                                                           int nvar, int nsub, int parity, int t0,
+                                                                           int slot_base, int tape_s0) {
+  __shared__ T sm[lds_elems<T, TX, TY, NS, kMaxTm, MODE != kInterior>()];
+  tm_batch_body<T, TX, TY, NS, MODE>(vars, pre_in, pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0, sm);
 }
 
 // the interior form held to 64 VGPRs, as tm_tiled_in2
 template <typename T, int TX, int TY, int NS>
-__global__ __launch_bounds__(BLK_TM) __attribute__((amdgpu_waves_per_eu(8, 8))) void tm_batch_in2(
-    const TmBatchVar<T>* vars, const int* prefix, int nvar, int nsub, int parity, int t0, int slot_base,
-    int tape_s0) {
-  tm_batch_body<T, TX, TY, NS, false>(vars, prefix, nvar, nsub, parity, t0, slot_base, tape_s0);
+__global__ __launch_bounds__((Shape<TX, TY, NS, kMaxTm>::BLK)) __attribute__((amdgpu_waves_per_eu(8, 8))) void
+tm_batch_in2(const TmBatchVar<T>* vars, const int* pre_in, const int* pre_ring, int nvar, int nsub, int parity,
+             int t0, int slot_base, int tape_s0) {
+  __shared__ T sm[lds_elems<T, TX, TY, NS, kMaxTm, false>()];
+  tm_batch_body<T, TX, TY, NS, kInterior>(vars, pre_in, pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0, sm);
 }
 
 }  // namespace
@@ -650,44 +768,66 @@ TileMap make_map(int nx, int ny, int in_i0, int in_i1, int in_j0, int in_j1) {
   return m;
 }
 
-// The interior launch is the one the kernel timing hook measures; its
-// cell-steps are the interior tiles' cells times the substeps.
-template <typename P, typename K1, typename K2>
-int launch_pair(const TileMap& m, K1 kin, K2 kpml, hipStream_t s, long long tile_cells, int nsub) {
-  int n_in = (m.r1 - m.r0) * (m.c1 - m.c0);
-  int n_ring = m.R * m.C - n_in;
+// A launch whose tiles all find a CU of their own (at most kOneRound) covers
+// interior and ring together: their latency chains then run side by side
+// instead of one after the other (TM 256^2, 16x64x4 tiles: 31.8 us per 4
+// steps in two launches, 15.6 us in one).  Larger grids take two launches,
+// which lets the interior kernel keep its smaller register footprint (and two
+// workgroups per CU).  The interior (or common) launch is the one the kernel
+// timing hook measures, its cell-steps the cells of its tiles times the
+// substeps.
+constexpr int kOneRound = 256;
+
+template <typename KA, typename K1, typename K2>
+void launch_tiles(const TileMap& m, KA kall, K1 kin, K2 kpml, hipStream_t s, long long tile_cells, int nsub) {
+  const int n_in = (m.r1 - m.r0) * (m.c1 - m.c0), n = m.R * m.C, n_ring = n - n_in;
+  if (n <= kOneRound && n_in && n_ring) {
+    timing_begin(s);
+    kall(dim3(n));
+    timing_end(s, (long long)n * tile_cells * nsub);
+    return;
+  }
   if (n_in) {
     timing_begin(s);
-    kin(dim3(m.c1 - m.c0, m.r1 - m.r0));
+    kin(dim3(n_in));
     timing_end(s, (long long)n_in * tile_cells * nsub);
   }
   if (n_ring) kpml(dim3(n_ring));
-  return MT_OK;
 }
 
 template <typename T, int TX, int TY, int NS>
 int launch_te_tiled(TeTiled<T> p, const TapSet& taps, int nsub, int write_e, hipStream_t s) {
+  constexpr int MI = te_max<TX, TY, NS>(false), MR = te_max<TX, TY, NS>(true);
   p.map = make_map<TX, TY, NS>(p.nx, p.ny, p.in_i0, p.in_i1, p.in_j0, p.in_j1);
-  launch_pair<T>(
+  launch_tiles(
       p.map,
-      [&](dim3 g) { hipLaunchKernelGGL((te_tiled<T, TX, TY, NS, false>), g, dim3(te_block(false)), 0, s, p, taps, nsub, write_e); },
-      [&](dim3 g) { hipLaunchKernelGGL((te_tiled<T, TX, TY, NS, true>), g, dim3(te_block(true)), 0, s, p, taps, nsub, write_e); },
+      [&](dim3 g) {
+        hipLaunchKernelGGL((te_tiled<T, TX, TY, NS, MR, kAll>), g, dim3(Shape<TX, TY, NS, MR>::BLK), 0, s, p, taps, nsub, write_e);
+      },
+      [&](dim3 g) {
+        hipLaunchKernelGGL((te_tiled<T, TX, TY, NS, MI, kInterior>), g, dim3(Shape<TX, TY, NS, MI>::BLK), 0, s, p, taps, nsub, write_e);
+      },
+      [&](dim3 g) {
+        hipLaunchKernelGGL((te_tiled<T, TX, TY, NS, MR, kRing>), g, dim3(Shape<TX, TY, NS, MR>::BLK), 0, s, p, taps, nsub, write_e);
+      },
       s, (long long)TX * TY, nsub);
   return check_launch("te2d tiled step");
 }
 
 template <typename T, int TX, int TY, int NS>
 int launch_tm_tiled(TmTiled<T> p, const TapSet& taps, int nsub, int tape_s0, hipStream_t s) {
+  constexpr int BLK = Shape<TX, TY, NS, kMaxTm>::BLK;
   p.map = make_map<TX, TY, NS>(p.nx, p.ny, p.in_i0, p.in_i1, p.in_j0, p.in_j1);
-  launch_pair<T>(
+  launch_tiles(
       p.map,
+      [&](dim3 g) { hipLaunchKernelGGL((tm_tiled<T, TX, TY, NS, kAll>), g, dim3(BLK), 0, s, p, taps, nsub, tape_s0); },
       [&](dim3 g) {
         if constexpr (sizeof(T) == 4)
-          hipLaunchKernelGGL((tm_tiled_in2<T, TX, TY, NS>), g, dim3(BLK_TM), 0, s, p, taps, nsub, tape_s0);
+          hipLaunchKernelGGL((tm_tiled_in2<T, TX, TY, NS>), g, dim3(BLK), 0, s, p, taps, nsub, tape_s0);
         else
-          hipLaunchKernelGGL((tm_tiled<T, TX, TY, NS, false>), g, dim3(BLK_TM), 0, s, p, taps, nsub, tape_s0);
+          hipLaunchKernelGGL((tm_tiled<T, TX, TY, NS, kInterior>), g, dim3(BLK), 0, s, p, taps, nsub, tape_s0);
       },
-      [&](dim3 g) { hipLaunchKernelGGL((tm_tiled<T, TX, TY, NS, true>), g, dim3(BLK_TM), 0, s, p, taps, nsub, tape_s0); },
+      [&](dim3 g) { hipLaunchKernelGGL((tm_tiled<T, TX, TY, NS, kRing>), g, dim3(BLK), 0, s, p, taps, nsub, tape_s0); },
       s, (long long)TX * TY, nsub);
   return check_launch("tm2d tiled step");
 }
@@ -696,19 +836,28 @@ template <typename T, int TX, int TY, int NS>
 int launch_tm_batch(const TmBatchVar<T>* vars, const int* pre_in, const int* pre_ring, int nvar, int n_in,
                     int n_ring, int grid_in, int grid_ring, int nsub, int parity, int t0, int slot_base,
                     int tape_s0, hipStream_t s) {
+  constexpr int BLK = Shape<TX, TY, NS, kMaxTm>::BLK;
+  const int n = n_in + n_ring;
+  if (n <= kOneRound && n_in && n_ring) {
+    timing_begin(s);
+    hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, kAll>), dim3(n), dim3(BLK), 0, s, vars, pre_in, pre_ring, nvar,
+                       nsub, parity, t0, slot_base, tape_s0);
+    timing_end(s, (long long)n * TX * TY * nsub);
+    return check_launch("tm2d batched step");
+  }
   if (n_in) {
     timing_begin(s);
     if constexpr (sizeof(T) == 4)
-      hipLaunchKernelGGL((tm_batch_in2<T, TX, TY, NS>), dim3(std::min(n_in, grid_in)), dim3(BLK_TM), 0, s, vars,
-                         pre_in, nvar, nsub, parity, t0, slot_base, tape_s0);
+      hipLaunchKernelGGL((tm_batch_in2<T, TX, TY, NS>), dim3(std::min(n_in, grid_in)), dim3(BLK), 0, s, vars,
+                         pre_in, pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0);
     else
-      hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, false>), dim3(std::min(n_in, grid_in)), dim3(BLK_TM), 0, s, vars,
-                       pre_in, nvar, nsub, parity, t0, slot_base, tape_s0);
+      hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, kInterior>), dim3(std::min(n_in, grid_in)), dim3(BLK), 0, s, vars,
+                         pre_in, pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0);
     timing_end(s, (long long)n_in * TX * TY * nsub);
   }
   if (n_ring)
-    hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, true>), dim3(std::min(n_ring, grid_ring)), dim3(BLK_TM), 0, s, vars,
-                       pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0);
+    hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, kRing>), dim3(std::min(n_ring, grid_ring)), dim3(BLK), 0, s, vars,
+                       pre_in, pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0);
   return check_launch("tm2d batched step");
 }
 
@@ -717,17 +866,27 @@ TileMap map_for(int nx, int ny, int in_i0, int in_i1, int in_j0, int in_j1) {
   return make_map<TX, TY, NS>(nx, ny, in_i0, in_i1, in_j0, in_j1);
 }
 
-// Tile-shape variants the autotuner chooses from (index = variant id).
-// (TX, TY, NS): owned rows, owned columns, Yee steps per launch.  FP64 tiles
-// are smaller so LDS (fields + psi) fits one workgroup.
+// Tile-shape variants (index = variant id), (TX, TY, NS): owned rows, owned
+// columns, Yee steps per launch.  FP64 tiles are smaller so that registers
+// and LDS fit one workgroup.  Variants 0-6 are for grids that fill the chip;
+// 7 on are for grids that do not: there a launch lasts as long as one tile
+// (VALU issue of the tile's cells on one CU, about 0.3 us per half-step and
+// 1000 cells, over about 6 us of launch, load and store latency), so the
+// smallest tile that still gives every tile its own CU wins, with as many
+// steps per launch as one cell per thread allows.  Measured per Yee step, TM
+// FP32: 256^2 16x16x7 2.2 us, 16x64x4 3.9 us; 100x60 8x8x8 2.0 us, 16x16x7
+// 2.2 us; 300^2 16x32x4 3.7 us, 16x64x4 3.9 us, 16x16x7 (361 tiles) 3.8 us.
 #define MT_VARIANTS_F32(X, T) \
-  X(T, 16, 64, 1) X(T, 16, 64, 2) X(T, 16, 64, 4) X(T, 32, 64, 1) X(T, 32, 64, 2) X(T, 32, 64, 4) X(T, 8, 128, 2)
+  X(T, 16, 64, 1) X(T, 16, 64, 2) X(T, 16, 64, 4) X(T, 32, 64, 1) X(T, 32, 64, 2) X(T, 32, 64, 4) X(T, 8, 128, 2) \
+  X(T, 16, 16, 7) X(T, 8, 8, 8) X(T, 16, 32, 4)
 #define MT_VARIANTS_F64(X, T) \
-  X(T, 8, 64, 1) X(T, 8, 64, 2) X(T, 8, 64, 4) X(T, 16, 64, 1) X(T, 16, 64, 2) X(T, 16, 32, 2) X(T, 8, 128, 1)
-static const int kVarF32[7][3] = {{16, 64, 1}, {16, 64, 2}, {16, 64, 4}, {32, 64, 1},
-                                  {32, 64, 2}, {32, 64, 4}, {8, 128, 2}};
-static const int kVarF64[7][3] = {{8, 64, 1}, {8, 64, 2}, {8, 64, 4}, {16, 64, 1},
-                                  {16, 64, 2}, {16, 32, 2}, {8, 128, 1}};
+  X(T, 8, 64, 1) X(T, 8, 64, 2) X(T, 8, 64, 4) X(T, 16, 64, 1) X(T, 16, 64, 2) X(T, 16, 32, 2) X(T, 8, 128, 1) \
+  X(T, 16, 16, 6) X(T, 8, 8, 8) X(T, 16, 32, 4)
+constexpr int kVariants = 10;
+static const int kVarF32[kVariants][3] = {{16, 64, 1}, {16, 64, 2}, {16, 64, 4}, {32, 64, 1}, {32, 64, 2},
+                                          {32, 64, 4}, {8, 128, 2}, {16, 16, 7}, {8, 8, 8}, {16, 32, 4}};
+static const int kVarF64[kVariants][3] = {{8, 64, 1}, {8, 64, 2}, {8, 64, 4}, {16, 64, 1}, {16, 64, 2},
+                                          {16, 32, 2}, {8, 128, 1}, {16, 16, 6}, {8, 8, 8}, {16, 32, 4}};
 
 int te_tiled_dispatch_f32(int variant, const TeTiled<float>& p, const TapSet& taps, int nsub, int write_e,
                           hipStream_t s) {
@@ -808,10 +967,10 @@ TileMap tiled_map(int variant, int dtype, int nx, int ny, int in_i0, int in_i1, 
   return TileMap{};
 }
 
-int tiled_variant_count() { return 7; }
+int tiled_variant_count() { return kVariants; }
 
 int tiled_variant_steps(int variant, int dtype) {
-  if (variant < 0 || variant >= 7) return 0;
+  if (variant < 0 || variant >= kVariants) return 0;
   return dtype == MT_F64 ? kVarF64[variant][2] : kVarF32[variant][2];
 }
 
@@ -819,10 +978,10 @@ int tiled_variant_steps(int variant, int dtype) {
 
 extern "C" int mt_tiled_variants(int dtype, int* steps, int* tx, int* ty) {
   const int(*tab)[3] = dtype == MT_F64 ? mt::kVarF64 : mt::kVarF32;
-  for (int v = 0; v < 7; ++v) {
+  for (int v = 0; v < mt::kVariants; ++v) {
     if (steps) steps[v] = tab[v][2];
     if (tx) tx[v] = tab[v][0];
     if (ty) ty[v] = tab[v][1];
   }
-  return 7;
+  return mt::kVariants;
 }

@@ -776,7 +776,7 @@ struct DispF64 {
 bool taps_ok(const MonitorPlan& mp) {
   for (int i = 0; i < mp.n_mons; ++i)
     for (int q = 0; q < mp.mons[i].n_terms; ++q)
-      if (mp.mons[i].term[q].line == 0) return false;
+      if (mp.mons[i].term[q].line == 0 || (mp.mons[i].term[q].field >= 3 && mp.mons[i].term[q].b)) return false;
   return true;
 }
 

@@ -24,6 +24,7 @@ import torch
 from . import _engine as E
 from .core import engine2d
 from .core.stepper_tm import FIELDS
+from .tune import one_round
 
 _ORDER = engine2d.TM_ORDER
 
@@ -96,8 +97,13 @@ class BatchedTM:
         E.require_device(c0.eps_inf)
         self.code = E.dtype_code(self.dtype)
         if variant is None:
-            # FP32: 32 x 64 tiles, 4 steps per launch (13% faster on C4 than 16 x 64)
-            variant = 5 if self.dtype == torch.float32 else 1
+            # the smallest tile with which the batch makes one round of
+            # workgroups; larger batches: 32 x 64 tiles, 4 steps per launch in
+            # FP32 (13% faster on 64 variants of 514^2 - 1522^2 than 16 x 64),
+            # 8 x 64 in FP64
+            variant = one_round(self.dtype, [tuple(p[0].eps_inf.shape) for p in problems])
+            if variant is None:
+                variant = 5 if self.dtype == torch.float32 else 2
         self.variant = int(variant)
         self.S = int(stage_steps)
         self.adjoint = bool(adjoint)

@@ -1,10 +1,13 @@
-"""Autotuner for the temporally blocked 2D steppers.
+"""Tile choice for the temporally blocked 2D steppers.
 
-For each problem signature (mode, grid, dtype, monitor layout) the first run
-times every tile variant (owned tile shape x Yee steps per launch, see
-mt_tiled_variants) and the two-pass per-half-step path on scratch copies of
-the real state, sources and monitors, and caches the fastest for the rest of
-the process.  MEEP_TORCH_AMD_VARIANT=<v> forces a variant (-1 = two-pass)."""
+A grid that fits the chip in one round of workgroups takes the smallest tile
+that does (`one_round`): its launch lasts as long as one tile, so fewer cells
+per tile and more steps per launch win.  Larger grids time the two large tile
+shapes on scratch copies of the real state, sources and monitors, once per
+problem signature (mode, grid, dtype, monitor layout), and cache the faster
+for the rest of the process; `tune` times any set of variants, the two-pass
+per-half-step path (-1) included.  MEEP_TORCH_AMD_VARIANT=<v> forces a variant
+(-1 = two-pass)."""
 import os
 
 import torch
@@ -12,9 +15,13 @@ import torch
 from . import _engine as E
 
 _CACHE = {}
-MIN_CELLS = 96 * 96          # below this, launch overhead dominates: no tuning
 TUNE_STEPS = 24
-DEFAULT_VARIANT = 1
+# variants from the smallest tile to the largest (mt_tiled_variants), and the
+# two timed on grids of more than one round.  Four steps or fewer do not repay
+# the tiled path's second buffer set.
+LADDER = {torch.float32: (8, 7, 9, 2, 5), torch.float64: (8, 7, 9, 2)}
+LARGE = {torch.float32: (2, 5), torch.float64: (2, 9)}
+ROUND = 256                  # compute units: tiles that run side by side
 
 
 def variants(dtype):
@@ -27,6 +34,17 @@ def variants(dtype):
     return [(int(tx[v]), int(ty[v]), int(steps[v])) for v in range(n)]
 
 
+def one_round(dtype, grids):
+    """The smallest tile with which the (nx, ny) grids together make at most
+    one round of workgroups; None if none does."""
+    shapes = variants(dtype)
+    for v in LADDER[dtype]:
+        tx, ty, _ = shapes[v]
+        if sum(-(-nx // tx) * -(-ny // ty) for nx, ny in grids) <= ROUND:
+            return v
+    return None
+
+
 def _key(mode, fields, monitors):
     ref = fields["Ez"] if mode == "tm" else fields["Hz"]
     return (mode, tuple(ref.shape), ref.dtype, ref.device.index,
@@ -37,20 +55,27 @@ def variant_for(mode, fields, coeffs, plan, monitors, k):
     env = os.environ.get("MEEP_TORCH_AMD_VARIANT")
     if env is not None:
         return int(env)
+    if k <= 4:
+        return -1
     ref = fields["Ez"] if mode == "tm" else fields["Hz"]
-    if ref.numel() < MIN_CELLS or k < 2 * TUNE_STEPS:
-        return DEFAULT_VARIANT
+    v = one_round(ref.dtype, [tuple(ref.shape)])
+    if v is not None:
+        return v
+    if k < 2 * TUNE_STEPS:
+        return LARGE[ref.dtype][0]
     key = _key(mode, fields, monitors)
     if key not in _CACHE:
-        _CACHE[key] = tune(mode, fields, coeffs, plan, monitors)
+        _CACHE[key] = tune(mode, fields, coeffs, plan, monitors, cands=LARGE[ref.dtype])
     return _CACHE[key]
 
 
-def tune(mode, fields, coeffs, plan, monitors, steps=TUNE_STEPS):
-    """Time each candidate on copies of `fields`; returns the fastest variant."""
+def tune(mode, fields, coeffs, plan, monitors, steps=TUNE_STEPS, cands=None):
+    """Time each candidate (default: every variant and the two-pass path) on
+    copies of `fields`; returns the fastest."""
     from .core import engine2d
     ref = fields["Ez"] if mode == "tm" else fields["Hz"]
-    cands = [-1] + list(range(len(variants(ref.dtype))))
+    if cands is None:
+        cands = [-1] + list(range(len(variants(ref.dtype))))
     times = {}
     for v in cands:
         work = {f: t.clone() for f, t in fields.items()}
