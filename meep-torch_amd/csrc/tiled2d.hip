@@ -254,6 +254,11 @@ __device__ __forceinline__ void te_tile(const TeTiled<T>& p, const TapSet& taps,
   const int tid = threadIdx.x, l0 = tid / RY, lj = tid - l0 * RY;
   const int i0 = a0 + l0, j = b0 + lj;
   const T dt = p.dt, dx = p.dx, rdx = p.rdx;
+  // shell rows, by value: read through p in the sub-step loop, a batched
+  // launch (p in device memory) would load them again after every store
+  const int hx_lo = p.hx.lo_end, hx_hi = p.hx.hi_begin, ex_lo = p.ex.lo_end + 1, ex_hi = p.ex.hi_begin + 1;
+  auto in_hx = [&](int i) { return i < hx_lo || i >= hx_hi; };
+  auto in_ex = [&](int i) { return i < ex_lo || i >= ex_hi; };
   auto ok = [&](int u) { return tid < STR && (u < PER - 1 || l0 + u * ROWS < RX); };
   const bool jhz = j >= 0 && j < ny - 1, jex = j >= 0 && j < ny;   // columns of Hz / Ey and of Ex
   const bool jin = j >= 1 && j < ny - 1;
@@ -277,8 +282,8 @@ __device__ __forceinline__ void te_tile(const TeTiled<T>& p, const TapSet& taps,
     vKy[u] = ey ? p.eps_y[(long long)i * (ny - 1) + j] : T(1);
     if constexpr (PML) {
       vPzy[u] = dget(p.pHzy, (long long)i * (ny - 2) + (j - 1), ex && in_ey);
-      vPzx[u] = dget(p.pHzx, (long long)(i - 1) * (ny - 1) + j, ey && i >= 1 && i < nx - 1 && p.ex.in(i - 1));
-      vPyx[u] = dget(p.pEyx, (long long)i * (ny - 1) + j, hz && p.hx.in(i));
+      vPzx[u] = dget(p.pHzx, (long long)(i - 1) * (ny - 1) + j, ey && i >= 1 && i < nx - 1 && in_ex(i));
+      vPyx[u] = dget(p.pEyx, (long long)i * (ny - 1) + j, hz && in_hx(i));
       vPxy[u] = dget(p.pExy, (long long)i * (ny - 1) + j, hz && in_hy);
     }
   }
@@ -319,7 +324,7 @@ __device__ __forceinline__ void te_tile(const TeTiled<T>& p, const TapSet& taps,
             vPzy[u] = ps;
             cx = cx + ps;
           }
-          if (jhz && (u > 0 || l0 >= 1) && i >= 1 && i < nx - 1 && p.ex.in(i - 1)) {
+          if (jhz && (u > 0 || l0 >= 1) && i >= 1 && i < nx - 1 && in_ex(i)) {
             const T ps = prof[2 * RX + li] * vPzx[u] + prof[3 * RX + li] * cy;
             vPzx[u] = ps;
             cy = cy + ps;
@@ -357,7 +362,7 @@ __device__ __forceinline__ void te_tile(const TeTiled<T>& p, const TapSet& taps,
         T a1 = qy[u];
         if constexpr (PML) {
           const bool h = lj < RY - 1 && li < RX - 1 && jhz && i >= 0 && i < nx - 1;
-          if (h && p.hx.in(i)) {
+          if (h && in_hx(i)) {
             const T ps = prof[li] * vPyx[u] + prof[RX + li] * qy[u];
             vPyx[u] = ps;
             a1 = a1 + ps;
@@ -405,7 +410,7 @@ __device__ __forceinline__ void te_tile(const TeTiled<T>& p, const TapSet& taps,
     if (i < nx - 1 && j < ny - 1) {
       p.oHz[h] = vHz[u];
       if constexpr (PML) {
-        if (p.hx.in(i)) p.oEyx[h] = vPyx[u];
+        if (in_hx(i)) p.oEyx[h] = vPyx[u];
         if (in_hy) p.oExy[h] = vPxy[u];
       }
     }
@@ -419,7 +424,7 @@ __device__ __forceinline__ void te_tile(const TeTiled<T>& p, const TapSet& taps,
       p.oDy[h] = vDy[u];
       if (write_e) p.Ey[h] = vEy[u];
       if constexpr (PML)
-        if (i >= 1 && i < nx - 1 && p.ex.in(i - 1)) p.oHzx[(long long)(i - 1) * (ny - 1) + j] = vPzx[u];
+        if (i >= 1 && i < nx - 1 && in_ex(i)) p.oHzx[(long long)(i - 1) * (ny - 1) + j] = vPzx[u];
     }
   }
 }
@@ -441,6 +446,11 @@ __device__ __forceinline__ void tm_tile(const TmTiled<T>& p, const TapSet& taps,
   const int tid = threadIdx.x, l0 = tid / RY, lj = tid - l0 * RY;
   const int i0 = a0 + l0, j = b0 + lj, jj = j - (p.y_pmc ? 0 : 1);
   const T dt = p.dt, dx = p.dx, rdx = p.rdx;
+  // shell rows, by value: read through p in the sub-step loop, a batched
+  // launch (p in device memory) would load them again after every store
+  const int hx_lo = p.hx.lo_end, hx_hi = p.hx.hi_begin, ex_lo = p.ex.lo_end + 1, ex_hi = p.ex.hi_begin + 1;
+  auto in_hx = [&](int i) { return i < hx_lo || i >= hx_hi; };
+  auto in_ex = [&](int i) { return i < ex_lo || i >= ex_hi; };
   auto ok = [&](int u) { return tid < STR && (u < PER - 1 || l0 + u * ROWS < RX); };
   const bool jez = j >= 0 && j < ny, jhx = j >= 0 && j < ny - 1;
   const bool jlive = jez && jj >= 0 && jj < ny_e;   // columns the D half updates
@@ -466,8 +476,8 @@ __device__ __forceinline__ void tm_tile(const TmTiled<T>& p, const TapSet& taps,
       const bool live = ez && i >= 1 && i < nx - 1 && jlive;
       const long long q = (long long)(i - 1) * ny_e + jj;
       vPzy[u] = dget(p.pEzy, (long long)i * (ny - 1) + j, hx && in_hy);
-      vPzx[u] = dget(p.pEzx, e, hy && p.hx.in(i));
-      vPyx[u] = dget(p.pHyx, q, live && p.ex.in(i - 1));
+      vPzx[u] = dget(p.pEzx, e, hy && in_hx(i));
+      vPyx[u] = dget(p.pHyx, q, live && in_ex(i));
       vPxy[u] = dget(p.pHxy, q, live && in_ey);
     }
   }
@@ -486,13 +496,15 @@ __device__ __forceinline__ void tm_tile(const TmTiled<T>& p, const TapSet& taps,
   const bool hx_tile = box_touches(p.hsrc[0], a0, b0, RX, RY), hy_tile = box_touches(p.hsrc[1], a0, b0, RX, RY);
   const bool tap_tile = taps.n && taps_touch(taps, I0, J0, TX, TY);
   const bool tap_d = tap_tile && taps_have(taps, 3);
+  const T *coef_tab = p.coef_tab, *hcoef_tab = p.hcoef_tab;
+  T* tape = p.tape;
   const bool jown = lj > NS && lj <= NS + TY && tid < STR && j < ny;
   auto own = [&](int u) {
     return jown && l0 + u * ROWS > NS && l0 + u * ROWS <= NS + TX && i0 + u * ROWS < nx;
   };
   for (int s = 0; s < nsub; ++s) {
-    const T coef = p.coef_tab ? p.coef_tab[coef_t0 + s] : p.coef[s];
-    const T hc = p.hcoef_tab ? p.hcoef_tab[coef_t0 + s] : p.hcoef[s];
+    const T coef = coef_tab ? coef_tab[coef_t0 + s] : p.coef[s];
+    const T hc = hcoef_tab ? hcoef_tab[coef_t0 + s] : p.hcoef[s];
     // B half (stepper_tm.py:85-92,126-128)
     {
       T qx[PER], qy[PER];
@@ -519,7 +531,7 @@ __device__ __forceinline__ void tm_tile(const TmTiled<T>& p, const TapSet& taps,
             vPzy[u] = ps;
             cy = cy + ps;
           }
-          if (jez && li < RX - 1 && i >= 0 && i < nx - 1 && p.hx.in(i)) {
+          if (jez && li < RX - 1 && i >= 0 && i < nx - 1 && in_hx(i)) {
             const T ps = prof[li] * vPzx[u] + prof[RX + li] * cx;
             vPzx[u] = ps;
             cx = cx + ps;
@@ -554,7 +566,7 @@ __device__ __forceinline__ void tm_tile(const TmTiled<T>& p, const TapSet& taps,
         T curl = qy[u];
         if constexpr (PML) {
           const bool live = lj >= 1 && (u > 0 || l0 >= 1) && jlive && i >= 1 && i < nx - 1;
-          if (live && p.ex.in(i - 1)) {
+          if (live && in_ex(i)) {
             const T ps = prof[2 * RX + li] * vPyx[u] + prof[3 * RX + li] * qy[u];
             vPyx[u] = ps;
             curl = curl + ps;
@@ -579,10 +591,10 @@ __device__ __forceinline__ void tm_tile(const TmTiled<T>& p, const TapSet& taps,
       }
     }
     __syncthreads();
-    if (p.tape) {
+    if (tape) {
 #pragma unroll
       for (int u = 0; u < PER; ++u)
-        if (own(u)) p.tape[(long long)(tape_s0 + s) * nx * ny + (long long)(i0 + u * ROWS) * ny + j] = vEz[u];
+        if (own(u)) tape[(long long)(tape_s0 + s) * nx * ny + (long long)(i0 + u * ROWS) * ny + j] = vEz[u];
     }
     if (tap_tile) {
       write_taps<T, RX, RY, 3>(
@@ -612,10 +624,10 @@ __device__ __forceinline__ void tm_tile(const TmTiled<T>& p, const TapSet& taps,
     if (i < nx - 1) p.oHy[e] = vHy[u];
     if constexpr (PML) {
       if (in_hy) p.oEzy[(long long)i * (ny - 1) + j] = vPzy[u];
-      if (i < nx - 1 && p.hx.in(i)) p.oEzx[e] = vPzx[u];
+      if (i < nx - 1 && in_hx(i)) p.oEzx[e] = vPzx[u];
       if (i >= 1 && i < nx - 1 && jlive) {
         const long long q = (long long)(i - 1) * ny_e + jj;
-        if (p.ex.in(i - 1)) p.oHyx[q] = vPyx[u];
+        if (in_ex(i)) p.oHyx[q] = vPyx[u];
         if (in_ey) p.oHxy[q] = vPxy[u];
       }
     }
