@@ -450,7 +450,7 @@ def bench_c4(args):
         gbs = alg * per_cells / per_s / 1e9
         adj_roof = {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": gbs / HBM_PEAK_GBS, "traffic": _traffic("c4_adjoint", per_cells),
-                    "kernel": "adj_batch_fused (one reverse step of every variant), HIP events on its stream",
+                    "kernel": "tm_reverse_batch (up to 4 reverse steps of every variant per launch), HIP events on its stream",
                     "launch_avg_us": per_s * 1e6, "cell_steps_per_launch": per_cells,
                     "alg_bytes_per_cell_update": alg}
     print(json.dumps({

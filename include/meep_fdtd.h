@@ -400,6 +400,19 @@ typedef struct {
 int mt_tm2d_adjoint(const mt_tm2d* p, const mt_tm2d_adj* a, const void* tape,
                     const mt_monitor* mons, int n_mons, int step0, int k, void* stream);
 
+/* The same reverse sweep, temporally blocked: several reverse steps per launch
+ * on overlapped tiles (p->variant: the forward's tile variant ids), for
+ * problems without media and symmetry cuts.  a holds the cotangents on entry
+ * and on return, b is a second set of the same shapes (its eps_grad and
+ * scratch are not read; nor are a's gHy..gEy).  Every monitor term needs its
+ * field position (mt_dft_term field, line, fix, lo); stage is a workspace of
+ * mt_stage_bytes(mons, n_mons, stage_steps, dtype) bytes into which the
+ * monitor cotangents of stage_steps steps are evaluated at a time.  Same
+ * results as mt_tm2d_adjoint. */
+int mt_tm2d_adjoint_tiled(const mt_tm2d* p, const mt_tm2d_adj* a, const mt_tm2d_adj* b, const void* tape,
+                          const mt_monitor* mons, int n_mons, void* stage, long long stage_bytes, int stage_steps,
+                          int step0, int k, void* stream);
+
 /* Adjoint state and scratch of one TE problem (same shapes as the forward
  * state; psi cotangents are tracked inside the CPML shells only). */
 typedef struct {
@@ -530,10 +543,10 @@ int mt_tm2d_batch_adjoint_sweep(mt_batch* b, int step0, int k, void* stream);
  * mt_tm2d_batch_adjoint_prepare): alt[v] has the same shapes as adj[v] and
  * the same eps_grad; mons are the monitor injections into that set (same
  * order and offsets).  When no variant has conductivity or ADE poles
- * (*fused = 1) every later sweep runs each reverse step as one fused pass
- * over tiles that reads one set and writes the other (the transposed
- * differences stay in LDS), and leaves the result in the first set; the
- * gradient is bit-identical to the three-pass sweep.  Same math as
+ * (*fused = 1) every later sweep runs several reverse steps per launch on
+ * overlapped tiles (as mt_tm2d_adjoint_tiled) that read one set and write the
+ * other, and leaves the result in the first set; the gradient is
+ * bit-identical to the three-pass sweep.  Same math as
  * mt_tm2d_batch_adjoint (the checkpointed backward of core/run.py:99-120). */
 int mt_tm2d_batch_adjoint_pingpong(mt_batch* b, const mt_tm2d_adj* alt, const mt_monitor* mons, const int* mon_off,
                                    int* fused, void* stream);

@@ -10,6 +10,7 @@
 
 #include "adjoint2d.h"
 #include "common.h"
+#include "reverse2d.h"
 #include "tiled2d.h"
 
 namespace {
@@ -19,7 +20,7 @@ constexpr int kCellBlk = 256;
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 struct Layout {
-  size_t vars, pre_in, pre_ring, adjk, adjk2, blk_pre, tile_pre, inj, inj2, inj_pre, tapes, dts, total;
+  size_t vars, pre_in, pre_ring, adjk, blk_pre, inj, inj_pre, tapes, dts, rev, rev_in, rev_ring, rev_stage, total;
 };
 
 template <typename T>
@@ -34,15 +35,9 @@ Layout layout(int nvar) {
   o = align256(o + (nvar + 1) * sizeof(int));
   L.adjk = o;
   o = align256(o + nvar * sizeof(mt::AdjK<T>));
-  L.adjk2 = o;
-  o = align256(o + nvar * sizeof(mt::AdjK<T>));
   L.blk_pre = o;
   o = align256(o + (nvar + 1) * sizeof(int));
-  L.tile_pre = o;
-  o = align256(o + (nvar + 1) * sizeof(int));
   L.inj = o;
-  o = align256(o + (size_t)kMaxMonPerVar * nvar * sizeof(mt_monitor));
-  L.inj2 = o;
   o = align256(o + (size_t)kMaxMonPerVar * nvar * sizeof(mt_monitor));
   L.inj_pre = o;
   o = align256(o + (size_t)kMaxMonPerVar * (nvar + 1) * sizeof(int));
@@ -50,6 +45,14 @@ Layout layout(int nvar) {
   o = align256(o + nvar * sizeof(void*));
   L.dts = o;
   o = align256(o + nvar * sizeof(double));
+  L.rev = o;
+  o = align256(o + nvar * sizeof(mt::TmRevVar<T>));
+  L.rev_in = o;
+  o = align256(o + (nvar + 1) * sizeof(int));
+  L.rev_ring = o;
+  o = align256(o + (nvar + 1) * sizeof(int));
+  L.rev_stage = o;
+  o = align256(o + (size_t)kMaxMonPerVar * nvar * sizeof(void*));
   L.total = o;
   return L;
 }
@@ -68,11 +71,13 @@ struct mt_batch {
   bool adj_ready = false;
   int adj_max_m = 0;
   std::vector<int> adj_inj_blocks;
-  // second cotangent set of the fused adjoint step (mt_tm2d_batch_adjoint_pingpong)
-  bool adj_fused = false;
-  int fused_tiles = 0;
+  // second cotangent set (mt_tm2d_batch_adjoint_pingpong)
   long long total_cells = 0;
   std::vector<mt_tm2d_adj> adj0, adj1;
+  std::vector<void*> tapes;
+  // temporally blocked reverse sweep over both sets (reverse2d.hip)
+  bool adj_tiled = false;
+  int rev_in = 0, rev_ring = 0;
 };
 
 namespace mt {
@@ -111,96 +116,6 @@ __global__ __launch_bounds__(kCellBlk) void adj_batch_inject(const mt_monitor* i
   const mt_monitor& m = inj[lo];
   if (m.n_terms == 0) return;
   adj_inject_block<T>(m, (b - pre[lo]) * kInjE, t, dts[lo], t_rel);
-}
-
-// Fused reverse step (no conductivity, no poles): one pass per tile of
-// FTI x FTJ cells of one variant.  A runs on the tile and a one-cell halo
-// (gHy on the rows above and below, gHx on the columns left and right),
-// B's Hy part on the tile and the row above, its Hx part on the tile and
-// the column to the left, C on the tile; gHy, gHx, gEx, gEy stay in LDS.
-// Every cotangent is read from set r (step t+1) and the tile's own cells
-// are written to set w (step t), so the halo reads never race with a
-// neighbour tile's writes; eps_grad (own cells only) is updated in place.
-// Same arithmetic as adj_a_cell / adj_b_cell / adj_c_cell.
-constexpr int FTI = 8, FTJ = 64;
-
-template <typename T>
-__global__ __launch_bounds__(FTI * FTJ) void adj_batch_fused(const AdjK<T>* rs, const AdjK<T>* wsd,
-                                                             void* const* tapes, const int* tile_pre, int nvar,
-                                                             int s_rel, int per_xcd) {
-  __shared__ T sGHy[FTI + 2][FTJ];   // rows i0-1 .. i0+FTI
-  __shared__ T sGHx[FTI][FTJ + 2];   // columns j0-1 .. j0+FTJ
-  __shared__ T sGEx[FTI + 1][FTJ];   // rows i0-1 .. i0+FTI-1
-  __shared__ T sGEy[FTI][FTJ + 1];   // columns j0-1 .. j0+FTJ-1
-  // XCD-aware order (as in tm_batch): XCD x takes the contiguous tile range
-  // [x * per_xcd, (x + 1) * per_xcd), so the tiles whose halos overlap share an L2
-  const int b = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if (b >= tile_pre[nvar]) return;
-  int lo = 0, hi = nvar;
-  while (hi - lo > 1) {
-    int mid = (lo + hi) >> 1;
-    if (tile_pre[mid] <= b) lo = mid;
-    else hi = mid;
-  }
-  const AdjK<T>& r = rs[lo];
-  const AdjK<T>& w = wsd[lo];
-  const int nx = r.nx, ny = r.ny;
-  const int ntj = (ny + FTJ - 1) / FTJ, t = b - tile_pre[lo];
-  const int i0 = (t / ntj) * FTI, j0 = (t % ntj) * FTJ;
-  const int tx = threadIdx.x, ty = threadIdx.y, q = ty * FTJ + tx;
-  const int i = i0 + ty, j = j0 + tx;
-  const bool own = i < nx && j < ny;
-  const T* ez_after = static_cast<const T*>(tapes[lo]) + (long long)s_rel * nx * ny;
-  // Every load of the A and B phases that does not depend on the A results
-  // is issued before the first store and barrier: the B inputs of the own
-  // cell and of this thread's B halo cell, then the A halo cell (which
-  // stores nothing), then the own A cell.
-  const bool hrow = q < FTJ, hcol = !hrow && q < FTJ + FTI;
-  const int rr = q - FTJ;
-  const BIn<T> pre = adj_b_load(r, i, j, own && i < nx - 1, own && j < ny - 1);
-  const BIn<T> preh = adj_b_load(r, hrow ? i0 - 1 : i0 + rr, hrow ? j0 + q : j0 - 1,
-                                 hrow && i0 >= 1 && j0 + q < ny, hcol && j0 >= 1 && i0 + rr < nx);
-  // ---- A
-  if (q < 2 * FTJ) {                      // rows i0-1 and i0+FTI: gHy
-    const int hi_row = q >= FTJ, jj = j0 + (q % FTJ), ii = hi_row ? i0 + FTI : i0 - 1;
-    T gy = T(0), gx;
-    if (ii >= 0 && ii < nx && jj < ny) adj_a_fused(r, w, ez_after, ii, jj, false, gy, gx);
-    sGHy[hi_row ? FTI + 1 : 0][q % FTJ] = gy;
-  } else if (q < 2 * FTJ + 2 * FTI) {     // columns j0-1 and j0+FTJ: gHx
-    const int q2 = q - 2 * FTJ, hi_col = q2 >= FTI, ii = i0 + (q2 % FTI), jj = hi_col ? j0 + FTJ : j0 - 1;
-    T gy, gx = T(0);
-    if (jj >= 0 && jj < ny && ii < nx) adj_a_fused(r, w, ez_after, ii, jj, false, gy, gx);
-    sGHx[q2 % FTI][hi_col ? FTJ + 1 : 0] = gx;
-  }
-  T ghy = T(0), ghx = T(0);
-  if (own) adj_a_fused(r, w, ez_after, i, j, true, ghy, ghx);
-  sGHy[ty + 1][tx] = ghy;
-  sGHx[ty][tx + 1] = ghx;
-  __syncthreads();
-  // ---- B
-  T gex = T(0), gey = T(0);
-  if (own && i < nx - 1) gex = adj_b_hy_pre(r, w, i, j, pre, sGHy[ty + 1][tx], sGHy[ty + 2][tx]);
-  if (own && j < ny - 1) gey = adj_b_hx_pre(r, w, i, j, pre, sGHx[ty][tx + 1], sGHx[ty][tx + 2]);
-  sGEx[ty + 1][tx] = gex;
-  sGEy[ty][tx + 1] = gey;
-  if (hrow) {                             // row i0-1: gEx
-    T g = T(0);
-    if (i0 >= 1 && j0 + q < ny) g = adj_b_hy_pre<T, false>(r, w, i0 - 1, j0 + q, preh, sGHy[0][q], sGHy[1][q]);
-    sGEx[0][q] = g;
-  } else if (hcol) {                      // column j0-1: gEy
-    T g = T(0);
-    if (j0 >= 1 && i0 + rr < nx) g = adj_b_hx_pre<T, false>(r, w, i0 + rr, j0 - 1, preh, sGHx[rr][0], sGHx[rr][1]);
-    sGEy[rr][0] = g;
-  }
-  __syncthreads();
-  // ---- C
-  if (own) {
-    const T gxm = i >= 1 ? sGEx[ty][tx] : T(0);
-    const T gx0 = i < nx - 1 ? sGEx[ty + 1][tx] : T(0);
-    const T gym = j >= 1 ? sGEy[ty][tx] : T(0);
-    const T gy0 = j < ny - 1 ? sGEy[ty][tx + 1] : T(0);
-    w.aEz[(long long)i * ny + j] = (gxm - gx0) / r.dx + (gym - gy0) / r.dx;
-  }
 }
 
 template <typename T>
@@ -361,110 +276,130 @@ int adjoint_prepare_t(mt_batch* b, const mt_tm2d_adj* adj, void* const* tapes, c
     return fail(MT_EHIP, "batched adjoint: descriptor upload failed");
   b->adj_max_m = max_m;
   b->adj0.assign(adj, adj + nvar);
-  b->adj_fused = false;
+  b->tapes.assign(tapes, tapes + nvar);
+  b->adj_tiled = false;
   b->adj_inj_blocks.assign(max_m, 0);
   for (int m = 0; m < max_m; ++m) b->adj_inj_blocks[m] = ipre[(size_t)m * (nvar + 1) + nvar];
   b->adj_ready = true;
   return MT_OK;
 }
 
-// Second cotangent set for the fused reverse step: descriptors of set 1
-// (same scratch and eps_grad as set 0) and monitor injections into it, plus
-// the tile prefix.  Applies when no variant has conductivity or poles;
-// *fused says whether the sweeps will use it.
+// Descriptors of the temporally blocked reverse sweep: both orientations of
+// the two cotangent sets, the monitor terms (staged in the variant's forward
+// staging buffer) and the tile prefixes.  *ok = false when a term has no
+// field position or a buffer is too small.
+template <typename T>
+int reverse_prepare_t(mt_batch* b, const mt_monitor* mons, const int* mon_off, bool* ok, hipStream_t s) {
+  *ok = false;
+  const int nvar = b->nvar;
+  std::vector<TmRevVar<T>> vars(nvar);
+  std::vector<int> pin(nvar + 1, 0), pring(nvar + 1, 0);
+  std::vector<void*> stage((size_t)kMaxMonPerVar * nvar, nullptr);
+  for (int v = 0; v < nvar; ++v) {
+    const mt_tm2d& d = b->probs[v];
+    const mt_monitor* mv = mons + mon_off[v];
+    const int nm = mon_off[v + 1] - mon_off[v];
+    MonitorPlan mp{mv, nm, b->stage[v], b->stage_bytes[v], b->S, b->dtype};
+    TmRevVar<T>& V = vars[v];
+    V.pA = make_rev<T>(&d, &b->adj0[v], &b->adj1[v], b->tapes[v]);
+    V.pB = make_rev<T>(&d, &b->adj1[v], &b->adj0[v], b->tapes[v]);
+    V.pB.eps_grad = V.pA.eps_grad;
+    V.pA.map = V.pB.map = rev_map(b->dtype, b->variant, d.nx, d.ny, V.pA.in_i0, V.pA.in_i1, V.pA.in_j0, V.pA.in_j1);
+    V.taps.n = 0;
+    if (nm) {
+      if (!rev_terms_ok(mv, nm) || mt_stage_bytes(mv, nm, b->S, b->dtype) > b->stage_bytes[v] || !b->stage[v] ||
+          !build_taps(mp, 0, 0, sizeof(T), &V.taps))
+        return MT_OK;
+      char* base = static_cast<char*>(b->stage[v]);
+      for (int m = 0; m < nm; ++m) {
+        if (mv[m].kind != 0) return MT_OK;
+        stage[(size_t)m * nvar + v] = base;
+        base += mt_stage_bytes(mv + m, 1, b->S, b->dtype);
+      }
+    }
+    const TileMap& m = V.pA.map;
+    const int n_in = (m.r1 - m.r0) * (m.c1 - m.c0);
+    pin[v + 1] = pin[v] + n_in;
+    pring[v + 1] = pring[v] + (m.R * m.C - n_in);
+  }
+  char* ws = b->ws;
+  if (hipMemcpyAsync(ws + b->L.rev, vars.data(), nvar * sizeof(TmRevVar<T>), hipMemcpyHostToDevice, s) ||
+      hipMemcpyAsync(ws + b->L.rev_in, pin.data(), (nvar + 1) * sizeof(int), hipMemcpyHostToDevice, s) ||
+      hipMemcpyAsync(ws + b->L.rev_ring, pring.data(), (nvar + 1) * sizeof(int), hipMemcpyHostToDevice, s) ||
+      hipMemcpyAsync(ws + b->L.rev_stage, stage.data(), stage.size() * sizeof(void*), hipMemcpyHostToDevice, s) ||
+      hipStreamSynchronize(s))
+    return fail(MT_EHIP, "batched adjoint: reverse descriptor upload failed");
+  b->rev_in = pin[nvar];
+  b->rev_ring = pring[nvar];
+  *ok = true;
+  return MT_OK;
+}
+
+// Reverse sweep with the temporally blocked tiles; ends in set 0.
+template <typename T>
+int reverse_sweep_t(mt_batch* b, int step0, int k, hipStream_t s) {
+  char* ws = b->ws;
+  const int nvar = b->nvar;
+  const int S = b->adj_max_m ? b->S : k;
+  const RevBatchArgs a{ws + b->L.rev, reinterpret_cast<const int*>(ws + b->L.rev_in),
+                       reinterpret_cast<const int*>(ws + b->L.rev_ring), nvar, b->variant, b->rev_in, b->rev_ring,
+                       b->grid_in};
+  const mt_monitor* inj = reinterpret_cast<const mt_monitor*>(ws + b->L.inj);
+  const int* dipre = reinterpret_cast<const int*>(ws + b->L.inj_pre);
+  const double* ddts = reinterpret_cast<const double*>(ws + b->L.dts);
+  void* const* stage = reinterpret_cast<void* const*>(ws + b->L.rev_stage);
+  int par = 0, rc;
+  for (const RevPart& part : rev_schedule(k, S, rev_steps(b->dtype, b->variant))) {
+    if (part.stage)
+      for (int m = 0; m < b->adj_max_m; ++m)
+        if (b->adj_inj_blocks[m])
+          rev_batch_stage<T>(inj + (size_t)m * nvar, stage + (size_t)m * nvar, dipre + (size_t)m * (nvar + 1),
+                             b->adj_inj_blocks[m], nvar, step0 + part.lo, part.stage, ddts, s);
+    timing_begin(s, 2);
+    rev_batch_run<T>(a, part, par, s);
+    timing_end(s, b->total_cells * part.nsub, 2);
+    par ^= 1;
+    if ((rc = check_launch("batched tm2d reverse sweep"))) return rc;
+  }
+  if (par)
+    for (int v = 0; v < nvar; ++v)
+      if ((rc = copy_cotangents(&b->probs[v], &b->adj0[v], &b->adj1[v], sizeof(T), s))) return rc;
+  return MT_OK;
+}
+
+// Second cotangent set for the temporally blocked reverse sweep: the
+// launches alternate between the two sets (set 0 again at the end).  Applies
+// when no variant has conductivity or poles; *fused says whether the sweeps
+// will use it.
 template <typename T>
 int adjoint_pingpong_t(mt_batch* b, const mt_tm2d_adj* alt, const mt_monitor* mons, const int* mon_off, int* fused,
                        hipStream_t s) {
   if (!b->adj_ready) return fail(MT_EINVAL, "batched adjoint: descriptors not prepared");
   const int nvar = b->nvar;
   *fused = 0;
-  b->adj_fused = false;
+  b->adj_tiled = false;
   for (int v = 0; v < nvar; ++v) {
     const mt_tm2d& d = b->probs[v];
     if (d.d1 || d.h1x || d.h1y || d.n_poles > 0) return MT_OK;
   }
-  std::vector<AdjK<T>> ks(nvar);
-  std::vector<int> tpre(nvar + 1, 0);
-  for (int v = 0; v < nvar; ++v) {
-    ks[v] = make_adjk<T>(&b->probs[v], &alt[v]);
-    const mt_tm2d& d = b->probs[v];
-    tpre[v + 1] = tpre[v] + ((d.nx + FTI - 1) / FTI) * ((d.ny + FTJ - 1) / FTJ);
-  }
-  std::vector<mt_monitor> inj((size_t)kMaxMonPerVar * nvar);
-  for (int m = 0; m < b->adj_max_m; ++m)
-    for (int v = 0; v < nvar; ++v) {
-      mt_monitor& dst = inj[(size_t)m * nvar + v];
-      dst = mt_monitor{};
-      if (m < mon_off[v + 1] - mon_off[v]) dst = mons[mon_off[v] + m];
-    }
-  char* ws = b->ws;
-  if (hipMemcpyAsync(ws + b->L.adjk2, ks.data(), nvar * sizeof(AdjK<T>), hipMemcpyHostToDevice, s) ||
-      hipMemcpyAsync(ws + b->L.tile_pre, tpre.data(), (nvar + 1) * sizeof(int), hipMemcpyHostToDevice, s) ||
-      hipMemcpyAsync(ws + b->L.inj2, inj.data(), inj.size() * sizeof(mt_monitor), hipMemcpyHostToDevice, s) ||
-      hipStreamSynchronize(s))
-    return fail(MT_EHIP, "batched adjoint: second-set upload failed");
   b->adj1.assign(alt, alt + nvar);
-  b->fused_tiles = tpre[nvar];
   b->total_cells = 0;
   for (int v = 0; v < nvar; ++v) b->total_cells += (long long)b->probs[v].nx * b->probs[v].ny;
-  b->adj_fused = true;
-  *fused = 1;
-  return MT_OK;
+  bool ok = false;
+  const int rc = reverse_prepare_t<T>(b, mons, mon_off, &ok, s);
+  b->adj_tiled = ok;
+  *fused = ok ? 1 : 0;
+  return rc;
 }
 
 // Reverse-time sweep over steps [step0, step0 + k) with the prepared
-// descriptors: per step, the monitor injection then either the fused pass
-// (alternating the two cotangent sets, set 0 again at the end) or the three
+// descriptors: the temporally blocked tiles over both cotangent sets, or,
+// without a second set, per step the monitor injection and the three
 // transpose passes over the cells of every variant.  Launches only.
 template <typename T>
 int adjoint_sweep_t(mt_batch* b, int step0, int k, hipStream_t s) {
   if (!b->adj_ready) return fail(MT_EINVAL, "batched adjoint: descriptors not prepared");
-  if (b->adj_fused) {
-    const int nvar = b->nvar;
-    char* ws = b->ws;
-    const AdjK<T>* k0 = reinterpret_cast<const AdjK<T>*>(ws + b->L.adjk);
-    const AdjK<T>* k1 = reinterpret_cast<const AdjK<T>*>(ws + b->L.adjk2);
-    void* const* dtp = reinterpret_cast<void* const*>(ws + b->L.tapes);
-    const int* tpre = reinterpret_cast<const int*>(ws + b->L.tile_pre);
-    const mt_monitor* inj0 = reinterpret_cast<const mt_monitor*>(ws + b->L.inj);
-    const mt_monitor* inj1 = reinterpret_cast<const mt_monitor*>(ws + b->L.inj2);
-    const int* dipre = reinterpret_cast<const int*>(ws + b->L.inj_pre);
-    const double* ddts = reinterpret_cast<const double*>(ws + b->L.dts);
-    int par = 0;
-    for (int s_ = k - 1; s_ >= 0; --s_) {
-      const int t = step0 + s_;
-      for (int m = 0; m < b->adj_max_m; ++m) {
-        const int nb = b->adj_inj_blocks[m];
-        if (nb)
-          hipLaunchKernelGGL(adj_batch_inject<T>, dim3(nb), dim3(kInjE * kInjS), 0, s,
-                             (par ? inj1 : inj0) + (size_t)m * nvar, dipre + (size_t)m * (nvar + 1), nvar, t, ddts,
-                             s_);
-      }
-      timing_begin(s, 2);
-      const int per_xcd = (b->fused_tiles + 7) / 8;
-      hipLaunchKernelGGL(adj_batch_fused<T>, dim3(8 * per_xcd), dim3(FTJ, FTI), 0, s, par ? k1 : k0,
-                         par ? k0 : k1, dtp, tpre, nvar, s_, per_xcd);
-      timing_end(s, b->total_cells, 2);
-      par ^= 1;
-      int rc = check_launch("batched tm2d fused adjoint step");
-      if (rc) return rc;
-    }
-    if (par) {  // odd step count: the cotangents are in set 1
-      for (int v = 0; v < nvar; ++v) {
-        const mt_tm2d& d = b->probs[v];
-        const mt_tm2d_adj &a0 = b->adj0[v], &a1 = b->adj1[v];
-        size_t nx = d.nx, ny = d.ny, nye = d.y_pmc ? d.ny : d.ny - 2;
-        size_t n[8] = {nx * ny, nx * ny, nx * (ny - 1), (nx - 1) * ny, nx * (ny - 1), (nx - 1) * ny,
-                       (nx - 2) * nye, (nx - 2) * nye};
-        void* dst[8] = {a0.aEz, a0.aDz, a0.aHx, a0.aHy, a0.apsi_Ezy, a0.apsi_Ezx, a0.apsi_Hyx, a0.apsi_Hxy};
-        void* src[8] = {a1.aEz, a1.aDz, a1.aHx, a1.aHy, a1.apsi_Ezy, a1.apsi_Ezx, a1.apsi_Hyx, a1.apsi_Hxy};
-        for (int q = 0; q < 8; ++q)
-          if (hipMemcpyAsync(dst[q], src[q], n[q] * sizeof(T), hipMemcpyDeviceToDevice, s) != hipSuccess)
-            return fail(MT_EHIP, "batched adjoint: copy back failed");
-      }
-    }
-    return MT_OK;
-  }
+  if (b->adj_tiled) return reverse_sweep_t<T>(b, step0, k, s);
   const int nvar = b->nvar;
   char* ws = b->ws;
   const AdjK<T>* dks = reinterpret_cast<const AdjK<T>*>(ws + b->L.adjk);

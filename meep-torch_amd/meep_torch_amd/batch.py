@@ -24,7 +24,7 @@ import torch
 from . import _engine as E
 from .core import engine2d
 from .core.stepper_tm import FIELDS
-from .tune import one_round
+from .tune import tile_for
 
 _ORDER = engine2d.TM_ORDER
 
@@ -84,7 +84,7 @@ class BatchedTM:
     def __init__(self, problems, n_steps, checkpoint_every=200, variant=None, stage_steps=64, adjoint=True,
                  fused_adjoint=True):
         self.L = E.lib()
-        # reverse steps as one fused pass over tiles with two cotangent sets
+        # reverse steps several per launch on tiles, with two cotangent sets
         # (False: the three transpose passes; the gradient is the same bit for bit)
         self.fused_adjoint = bool(fused_adjoint)
         _bind(self.L)
@@ -97,13 +97,7 @@ class BatchedTM:
         E.require_device(c0.eps_inf)
         self.code = E.dtype_code(self.dtype)
         if variant is None:
-            # the smallest tile with which the batch makes one round of
-            # workgroups; larger batches: 32 x 64 tiles, 4 steps per launch in
-            # FP32 (13% faster on 64 variants of 514^2 - 1522^2 than 16 x 64),
-            # 8 x 64 in FP64
-            variant = one_round(self.dtype, [tuple(p[0].eps_inf.shape) for p in problems])
-            if variant is None:
-                variant = 5 if self.dtype == torch.float32 else 2
+            variant = tile_for(self.dtype, [tuple(p[0].eps_inf.shape) for p in problems])
         self.variant = int(variant)
         self.S = int(stage_steps)
         self.adjoint = bool(adjoint)
@@ -334,8 +328,8 @@ class BatchedTM:
         off_arr = (E.c_int * (B + 1))(*off)
         rc = self.L.mt_tm2d_batch_adjoint_prepare(h, adjs, tapes, mon_arr, off_arr, E.stream_handle())
         E.check(rc, "mt_tm2d_batch_adjoint_prepare")
-        # second cotangent set: the fused reverse step reads one set and
-        # writes the other (batched variants carry no conductivity or poles)
+        # second cotangent set: the tiled reverse launches read one set and
+        # write the other (batched variants carry no conductivity or poles)
         fused = E.c_int(0)
         adjs2, mons2, keep2 = (E.TM2DAdj * B)(), [], []
         if self.fused_adjoint:

@@ -5,7 +5,8 @@ Replaces the reference's autograd through torch.utils.checkpoint chunks
 interval, saving the full TM state on the device every K steps (K =
 checkpoint_every, or 200).  Backward: for each chunk, last first, the chunk is
 recomputed from its checkpoint while a tape records Ez after every step, then
-mt_tm2d_adjoint sweeps the chunk backwards, injecting the monitor cotangents
+mt_tm2d_adjoint_tiled (several reverse steps per launch on tiles; with media or
+symmetry cuts mt_tm2d_adjoint, step by step) sweeps the chunk backwards, injecting the monitor cotangents
 dL/dacc and accumulating dL/deps = sum_t -(dL/dEz_t) Ez_t / eps.  The gradient
 reaches whatever graph produced eps_inf (filters, projection, paint) through
 autograd as usual.
@@ -23,6 +24,7 @@ import ctypes
 import torch
 
 from .. import _engine as E
+from .. import tune
 from . import engine2d
 from .stepper_te import fields_of as te_fields_of
 from .stepper_tm import fields_of as tm_fields_of
@@ -45,6 +47,8 @@ def _adj_monitors(adj_fields, monitors, gaccs, dtype, device):
             pa, s0, s1, n0, n1 = E.view2d(a)
             if q == 0:
                 m.n0, m.n1 = n0, n1
+            if len(term) > 3 and term[3] is not None:   # the term's field position (tile kernels)
+                m.term[q].field, m.term[q].line, m.term[q].fix, m.term[q].lo = term[3]
             m.term[q].a = pa
             m.term[q].b = E.view2d(b)[0] if b is not None else None
             m.term[q].s0, m.term[q].s1 = s0, s1
@@ -168,6 +172,17 @@ class _TMRun(torch.autograd.Function):
             extra["c3"] = torch.zeros(cdet.c3.shape, dtype=dtype, device=device)
             if cdet.c3.shape[0]:
                 a.c3_grad = extra["c3"].data_ptr()
+        # without media and cuts, when every monitor term has a field position:
+        # several reverse steps per launch on tiles, between two cotangent sets
+        tiled = not (kerr or cdet.d1 is not None or cdet.h1x is not None or cdet.c1.shape[0] or cdet.mc1x is not None
+                     or cdet.y_mirror_lo or cdet.x_mirror_lo) and \
+            all(len(t) > 3 and t[3] is not None for m in monitors for t in m.engine_terms(adj)[1])
+        if tiled:
+            d.variant = tune.tile_for(dtype, [(nx, ny)])
+            adj2 = {f: t.clone() for f, t in adj.items()}
+            a2 = E.TM2DAdj()
+            for f in names:
+                setattr(a2, "a" + f, adj2[f].data_ptr())
         for step0, k, st in reversed(ctx.ckpts):
             work = {f: t.clone() for f, t in st.items()}
             a.ez_init = st["Ez"].data_ptr()
@@ -175,9 +190,16 @@ class _TMRun(torch.autograd.Function):
             engine2d.run_chunk("tm", work, cdet, step0, k, plan, [], tape=tape)
             g_chunk = _chunk_cotangents(monitors, gacc, step0, k)
             arr, n_used, keep = _adj_monitors(adj, monitors, g_chunk, dtype, device)
-            rc = L.mt_tm2d_adjoint(ctypes.byref(d), ctypes.byref(a), E.ptr(tape), arr, n_used,
-                                   step0, k, E.stream_handle())
-            E.check(rc, "mt_tm2d_adjoint")
+            if tiled:
+                S, stage, nbytes = engine2d.stage_alloc(L, arr, n_used, E.dtype_code(dtype), device)
+                rc = L.mt_tm2d_adjoint_tiled(ctypes.byref(d), ctypes.byref(a), ctypes.byref(a2), E.ptr(tape), arr,
+                                             n_used, E.ptr(stage) if stage is not None else None, nbytes, S,
+                                             step0, k, E.stream_handle())
+                E.check(rc, "mt_tm2d_adjoint_tiled")
+            else:
+                rc = L.mt_tm2d_adjoint(ctypes.byref(d), ctypes.byref(a), E.ptr(tape), arr, n_used,
+                                       step0, k, E.stream_handle())
+                E.check(rc, "mt_tm2d_adjoint")
             del keep, tape
         del d_keep
         g_state = [adj[f] for f in names][:ctx.n_state]
