@@ -76,6 +76,61 @@ int mt_unpack_spectral_grad(const float* dwp, float* dwre, float* dwim, int Ci, 
 int mt_adam(float* w, const float* g, float* m, float* v, long long n, float lr, float b1, float b2, float eps,
             int step, float wd, void* stream);
 
+/* Fused passes of the operator with 64 channels, 128 modes, 128 head units and
+ * P = n*n points, P % 16 == 0 (matrix-core size; other sizes use the calls
+ * above).  Activations are (B, 64, P) BF16, spectra (B, 256, 64) BF16 with row
+ * 2 m + re/im, FP32 partial sums are folded in a fixed order.  16-byte aligned
+ * BF16 pointers.
+ *
+ * lift: x16 (B, 3, P) = [rho, (i+0.5)/n, (j+0.5)/n], v16 = w x16 + bias.
+ * lift_back: drho = w[:, 0]^T dv16. */
+int mt_fno_lift(const float* rho, const void* w, const float* bias, void* x16, void* v16, int B, int n,
+                void* stream);
+int mt_fno_lift_back(const void* dv16, const void* w, float* drho, int B, int P, void* stream);
+
+/* part (splits, B, 256, 64) = x16 against the 256 rows of basis (256, P), the
+ * points split in order; with y16 also wpart (splits, B, 64, 64) =
+ * sum_p x16[c'] y16[c]. */
+int mt_fno_dft(const void* x16, const void* basis, const void* y16, float* part, float* wpart, int B, int P,
+               int splits, void* stream);
+
+/* Per mode m: in16[b] = BF16 of the summed partials (row pair 2m, 2m+1: 128
+ * values), out16[b][n] = sum_k in16[b][k] w[m][n][k]. */
+int mt_fno_mix(const float* part, int splits, const void* w, void* in16, void* out16, int B, int Mo, void* stream);
+
+/* u = basis_t u16 + w (64 x 64) x16 + bias -> pre (if not NULL); y16 = gelu(u)
+ * or u.  basis_t: rows p of (P, 256) in fragment order, [ceil(P/128) * 4]
+ * 32-point tiles x [16] steps of 16 x [64] lanes x [8]: lane 32 h + i holds
+ * point 32 t + i, values 16 q + 8 h .. + 7. */
+int mt_fno_out(const void* u16, const void* basis_t, const void* w, const void* x16, const float* bias, float* pre,
+               void* y16, int B, int P, int act, void* stream);
+
+/* d = (basis_t u16 + w x16) (* gelu'(pre) with act) -> y16; part (B,
+ * ceil(P/128), 64) = sums of d over each 128 points (if not NULL). */
+int mt_fno_out_back(const void* u16, const void* basis_t, const void* w, const void* x16, const float* pre,
+                    void* y16, float* part, int B, int P, int act, void* stream);
+
+/* out = wo mean_P gelu(wq v16 + bq) + bo; part: scratch of B * chunks * 128. */
+int mt_fno_head(const void* v16, const void* wq, const float* bq, const void* wo, const float* bo, float* part,
+                int chunks, void* hm16, float* out, int B, int P, int n_out, void* stream);
+
+/* Backward of mt_fno_head: dv16; with dwo also dwo, dbo and the partial sums
+ * (B * chunks, ...) of dbq (128), of dv's channels (64) and of dwq (128, 64).
+ * wq_t (64, 128) is wq transposed. */
+int mt_fno_head_back(const float* dout, const void* v16, const void* wq, const void* wq_t, const float* bq,
+                     const void* wo, const void* hm16, float* dwo, float* dbo, float* dhm, void* dv16,
+                     float* qbpart, float* vbpart, float* qwpart, int chunks, int B, int P, int n_out,
+                     void* stream);
+
+/* out[i] = sum_{q<Q} part[q][i], i < n (part is overwritten). */
+int mt_fno_fold(float* part, int Q, int n, float* out, void* stream);
+
+/* mt_pack_spectral for Ci = Co = C, and its per-mode transpose wp_t. */
+int mt_fno_pack(const float* wre, const float* wim, void* wp, void* wp_t, int C, int Mo, void* stream);
+
+/* y (C, R) = BF16 of x (R, C) transposed. */
+int mt_transpose_bf16(const float* x, void* y, int R, int C, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -35,6 +35,21 @@ def lib():
     L.mt_unpack_spectral_grad.argtypes = [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]
     L.mt_adam.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_ll, c_float, c_float, c_float, c_float,
                           c_int, c_float, c_void_p]
+    V, I = c_void_p, c_int
+    L.mt_fno_lift.argtypes = [V, V, V, V, V, I, I, V]
+    L.mt_fno_lift_back.argtypes = [V, V, V, I, I, V]
+    L.mt_fno_dft.argtypes = [V, V, V, V, V, I, I, I, V]
+    L.mt_fno_mix.argtypes = [V, I, V, V, V, I, I, V]
+    L.mt_fno_out.argtypes = [V, V, V, V, V, V, V, I, I, I, V]
+    L.mt_fno_out_back.argtypes = [V, V, V, V, V, V, V, I, I, I, V]
+    L.mt_fno_head.argtypes = [V, V, V, V, V, V, I, V, V, I, I, I, V]
+    L.mt_fno_head_back.argtypes = [V] * 14 + [I, I, I, I, V]
+    L.mt_fno_fold.argtypes = [V, I, I, V, V]
+    L.mt_fno_pack.argtypes = [V, V, V, V, I, I, V]
+    L.mt_transpose_bf16.argtypes = [V, V, I, I, V]
+    for n in ("mt_fno_lift", "mt_fno_lift_back", "mt_fno_dft", "mt_fno_mix", "mt_fno_out", "mt_fno_out_back",
+              "mt_fno_head", "mt_fno_head_back", "mt_fno_fold", "mt_fno_pack", "mt_transpose_bf16"):
+        getattr(L, n).restype = c_int
     for n in ("mt_gemm_bf16", "mt_cast_bf16", "mt_bias_act", "mt_act_grad", "mt_channel_sum", "mt_row_sum",
               "mt_pack_spectral", "mt_unpack_spectral_grad", "mt_adam"):
         getattr(L, n).restype = c_int
@@ -140,3 +155,10 @@ def unpack_spectral_grad(dwp, dwre, dwim, Ci, Co, Mo):
 def adam(w, g, m, v, lr, b1, b2, eps, step, wd=0.0):
     E.check(lib().mt_adam(_p(w), _p(g), _p(m), _p(v), w.numel(), float(lr), float(b1), float(b2), float(eps),
                           int(step), float(wd), E.stream_handle()), "mt_adam")
+
+
+def fno(name, *args):
+    """Call mt_<name> of the fused operator passes: tensors as pointers, the
+    current stream last."""
+    a = [_p(x) if torch.is_tensor(x) or x is None else x for x in args]
+    E.check(getattr(lib(), "mt_" + name)(*a, E.stream_handle()), "mt_" + name)

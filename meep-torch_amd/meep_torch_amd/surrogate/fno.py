@@ -101,8 +101,23 @@ class SpectralOperator:
         self.GT = self._bf(np.ascontiguousarray(G.T))
         self.ws = _nn.Workspace(self.device)
         self._wbf = {}
+        # the fused passes' size (spectral.hip); their 128-bit loads need rows
+        # of whole 16-point groups
+        self.fused = (self.C == 64 and self.Mo == 128 and self.H == 128 and self.in_ch == 3 and self.P % 16 == 0)
+        if self.fused:
+            self.GTf, self.FTf = self._fragments(self.GT), self._fragments(self.FT)
         self.sync_weights()
         self._buf = {}
+
+    @staticmethod
+    def _fragments(t):
+        """(P, K) basis rows in the order the matrix cores take them: 32-point
+        tiles (P padded with zeros to whole 128-point tiles), 16-wide steps of
+        K, then lane = 32 * half + point with 8 values each."""
+        P, K = t.shape
+        pad = -P % 128
+        t = torch.cat([t, t.new_zeros(pad, K)]) if pad else t
+        return t.view(-1, 32, K // 16, 2, 8).permute(0, 2, 3, 1, 4).contiguous()
 
     # ---- parameters -------------------------------------------------------
     def _views(self, flat):
@@ -146,10 +161,18 @@ class SpectralOperator:
             if name not in self._wbf:
                 self._wbf[name] = torch.empty(t.shape, dtype=torch.bfloat16, device=self.device)
             _nn.cast_bf16(t, self._wbf[name])
+        if self.fused:   # also the transposes that the fused passes read along their reductions
+            for name, R, Q in [("q_w", self.H, C)] + [(f"w{l}", C, C) for l in range(self.L)]:
+                t = self._wbf.setdefault(name + "T", torch.empty((Q, R), dtype=torch.bfloat16, device=self.device))
+                _nn.fno("transpose_bf16", self.p[name], t, R, Q)
         for l in range(self.L):
             key = f"wp{l}"
             if key not in self._wbf:
                 self._wbf[key] = torch.empty((Mo, 2 * C, 2 * C), dtype=torch.bfloat16, device=self.device)
+            if self.fused:
+                t = self._wbf.setdefault(key + "T", torch.empty_like(self._wbf[key]))
+                _nn.fno("fno_pack", self.p[f"s{l}_re"], self.p[f"s{l}_im"], self._wbf[key], t, C, Mo)
+                continue
             _nn.pack_spectral(self.p[f"s{l}_re"], self.p[f"s{l}_im"], self._wbf[key], C, C, Mo)
 
     def state_dict(self):
@@ -188,6 +211,8 @@ class SpectralOperator:
         if rho.dim() != 3 or rho.shape[1:] != (self.n, self.n):
             raise ValueError(f"rho must be (B, {self.n}, {self.n})")
         rho = rho.detach().to(torch.float32).contiguous()
+        if self.fused:
+            return self._forward_fused(rho)
         B, C, P, Mo, H, L = rho.shape[0], self.C, self.P, self.Mo, self.H, self.L
         ws, W, bf, f32 = self.ws, self._wbf, torch.bfloat16, torch.float32
         CP, S = C * P, 2 * Mo * C
@@ -244,6 +269,8 @@ class SpectralOperator:
         CP, S = C * P, 2 * Mo * C
         b = self._buf
         dout = dout.detach().to(f32).contiguous()
+        if self.fused:
+            return self._backward_fused(dout, param_grads, input_grad)
         d16 = _nn.cast_bf16(dout, self._get("dout16", (B, n_out), bf))
         if param_grads:
             _nn.channel_sum(dout, g["o_b"], B, n_out, 1, ws=ws)
@@ -302,6 +329,95 @@ class SpectralOperator:
         drho = torch.empty((B, self.n, self.n), dtype=f32, device=self.device)
         _nn.gemm(W["lift_w"], (1, self.in_ch, 0, 0), dp16, (P, 1, CP, 0), drho, (P, 1, P), 1, P, C, batch=B,
                  ws=ws)
+        return drho
+
+    # ---- fused passes (spectral.hip) ----------------------------------------
+    def _splits(self, B):
+        """Reduction splits of the truncated DFT: about 512 workgroups (two per
+        CU) over the batch, at least 128 points each."""
+        return max(1, min(_nn.TARGET_WG // B, self.P // 128))
+
+    def _chunks(self, B):
+        """Workgroups per batch row of the head passes (128-point tiles, about
+        1024 workgroups in all)."""
+        return max(1, min(-(-self.P // 128), 1024 // B))
+
+    def _part(self, key, *shape):
+        """A view of a partial-sum buffer that grows to the largest call."""
+        n = int(np.prod(shape))
+        t = self._buf.get(key)
+        if t is None or t.numel() < n:
+            t = self._buf[key] = torch.empty(n, dtype=torch.float32, device=self.device)
+        return t[:n]
+
+    def _forward_fused(self, rho):
+        B, C, P, Mo, H, L = rho.shape[0], self.C, self.P, self.Mo, self.H, self.L
+        W, p, bf, f32, call = self._wbf, self.p, torch.bfloat16, torch.float32, _nn.fno
+        spec = (B, 2 * Mo, C)
+        v = self._get("v0", (B, C, P), bf)
+        call("fno_lift", rho, W["lift_w"], p["lift_b"], self._get("x16", (B, 3, self.n, self.n), bf), v, B, self.n)
+        sp = self._splits(B)
+        part = self._part("part", sp, B, 2 * Mo, C)
+        uh16 = self._get("uh16", spec, bf)
+        for l in range(L):
+            act = l < L - 1
+            call("fno_dft", v, self.F, None, part, None, B, P, sp)
+            call("fno_mix", part, sp, W[f"wp{l}T"], self._get(f"vh16_{l}", spec, bf), uh16, B, Mo)
+            pre = self._get(f"pre{l}", (B, C, P), f32) if act else None   # gelu' needs it, the last layer has none
+            vn = self._get(f"v{l + 1}", (B, C, P), bf)
+            call("fno_out", uh16, self.GTf, W[f"w{l}"], v, p[f"b{l}"], pre, vn, B, P, int(act))
+            v = vn
+        ch = self._chunks(B)
+        out = torch.empty((B, self.n_out), dtype=f32, device=self.device)
+        call("fno_head", v, W["q_w"], p["q_b"], W["o_w"], p["o_b"], self._part("hpart", B, ch, H), ch,
+             self._get("hm16", (B, H), bf), out, B, P, self.n_out)
+        self._saved_B = B
+        return out
+
+    def _backward_fused(self, dout, param_grads, input_grad):
+        B, C, P, Mo, H, L = self._saved_B, self.C, self.P, self.Mo, self.H, self.L
+        W, p, g, b, bf, f32, call = self._wbf, self.p, self.g, self._buf, torch.bfloat16, torch.float32, _nn.fno
+        spec, S, tiles = (B, 2 * Mo, C), 2 * Mo * C, -(-P // 128)
+        ch, sp = self._chunks(B), self._splits(B)
+        dp, dp_next = self._get("dp16", (B, C, P), bf), self._get("dp16b", (B, C, P), bf)
+        qb = vb = qw = None
+        if param_grads:
+            qb, vb, qw = (self._part(k, B, ch, n) for k, n in (("qbpart", H), ("vbpart", C), ("qwpart", H * C)))
+        call("fno_head_back", dout, b[f"v{L}"], W["q_w"], W["q_wT"], p["q_b"], W["o_w"], b["hm16"],
+             g["o_w"] if param_grads else None, g["o_b"] if param_grads else None, self._get("dhm", (B, H), f32), dp,
+             qb, vb, qw, ch, B, P, self.n_out)
+        if param_grads:
+            call("fno_fold", qb, B * ch, H, g["q_b"])
+            call("fno_fold", qw, B * ch, H * C, g["q_w"])
+            call("fno_fold", vb, B * ch, C, g[f"b{L - 1}"])
+        part = self._part("part", sp, B, 2 * Mo, C)
+        wpart = self._part("wpart", sp, B, C, C) if param_grads else None
+        bpart = self._part("bpart", B, tiles, C) if param_grads else None
+        duh16, dvh16 = self._get("duh16", spec, bf), self._get("dvh16", spec, bf)
+        for l in range(L - 1, -1, -1):
+            # dp: gradient of the layer's pre-activation.  Its spectrum against
+            # the inverse basis, and the pointwise weight gradient
+            call("fno_dft", dp, self.G, b[f"v{l}"] if param_grads else None, part, wpart, B, P, sp)
+            if param_grads:
+                call("fno_fold", wpart, sp * B, C * C, g[f"w{l}"])
+            call("fno_mix", part, sp, W[f"wp{l}"], duh16, dvh16, B, Mo)
+            if param_grads:
+                dwp = self._get("dwp", (Mo, 2 * C, 2 * C), f32)
+                _nn.gemm(b[f"vh16_{l}"], (1, S, 2 * C, 0), duh16, (S, 1, 2 * C, 0), dwp, (2 * C, 1, 4 * C * C),
+                         2 * C, 2 * C, B, batch=Mo, ws=self.ws)
+                _nn.unpack_spectral_grad(dwp, g[f"s{l}_re"], g[f"s{l}_im"], C, C, Mo)
+            if l == 0 and not input_grad:
+                return None
+            call("fno_out_back", dvh16, self.FTf, W[f"w{l}T"], dp, b[f"pre{l - 1}"] if l else None, dp_next, bpart, B,
+                 P, int(l > 0))
+            if param_grads:
+                call("fno_fold", bpart, B * tiles, C, g[f"b{l - 1}"] if l else g["lift_b"])
+            dp, dp_next = dp_next, dp
+        if param_grads:
+            _nn.gemm(dp, (P, 1, 0, C * P), b["x16"], (1, P, 0, 3 * P), g["lift_w"], (3, 1, 0), C, 3, P, R=B,
+                     ws=self.ws)
+        drho = torch.empty((B, self.n, self.n), dtype=f32, device=self.device)
+        call("fno_lift_back", dp, W["lift_w"], drho, B, P)
         return drho
 
     # ---- optimizer ----------------------------------------------------------
