@@ -22,8 +22,6 @@
 namespace mt {
 namespace {
 
-constexpr int BZ = 64;
-constexpr int BYY = 4;
 
 template <typename T>
 struct K3 {
@@ -154,9 +152,9 @@ __device__ __forceinline__ void h3_cell(const K3<T>& p, int i, int j, int k) {
 }
 
 template <typename T, bool M, bool A = false>
-__global__ __launch_bounds__(BZ* BYY) void h3_kernel(K3<T> p) {
-  const int k = blockIdx.x * BZ + threadIdx.x;
-  const int j = blockIdx.y * BYY + threadIdx.y;
+__global__ __launch_bounds__(kBlock3) void h3_kernel(K3<T> p) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  const int j = blockIdx.y * blockDim.y + threadIdx.y;
   if (j >= p.ny || k >= p.nz) return;
   h3_cell<T, M, A>(p, blockIdx.z, j, k);
 }
@@ -339,9 +337,9 @@ __device__ __forceinline__ void e3_cell(const K3<T>& p, const mt_source3d& src, 
 }
 
 template <typename T, bool M, bool A = false>
-__global__ __launch_bounds__(BZ* BYY) void e3_kernel(K3<T> p, mt_source3d src, T c, T* tape) {
-  const int k = blockIdx.x * BZ + threadIdx.x;
-  const int j = blockIdx.y * BYY + threadIdx.y;
+__global__ __launch_bounds__(kBlock3) void e3_kernel(K3<T> p, mt_source3d src, T c, T* tape) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  const int j = blockIdx.y * blockDim.y + threadIdx.y;
   if (j >= p.ny || k >= p.nz) return;
   e3_cell<T, M, A>(p, src, c, tape, blockIdx.z, j, k);
 }
@@ -1456,8 +1454,7 @@ int run3_tb2(const mt_yee3d* d, K3<T> p, const mt_source3d& sv, const double* co
   if (s_ < k) {   // odd count: the last step in place, two-pass
     void* const* A = in_alt ? B0 : A0;
     set_io(p, A, A);
-    dim3 blk(BZ, BYY, 1);
-    dim3 grd((nz + BZ - 1) / BZ, (ny + BYY - 1) / BYY, nx);
+    const dim3 blk = block3(ny, nz), grd = grid3(blk, nx, ny, nz);
     const T c = sv.kind ? static_cast<T>(coef[s_]) : T(0);
     hipLaunchKernelGGL((h3_kernel<T, false>), grd, blk, 0, s, p);
     hipLaunchKernelGGL((e3_kernel<T, false>), grd, blk, 0, s, p, sv, c, (T*)nullptr);
@@ -1531,8 +1528,7 @@ int run3_t(const mt_yee3d* d, const mt_source3d* src, const double* coef, const 
     }
     return run3_split<T, 4>(d, p, sv, coef, mp, step0, k, s);
   }
-  dim3 blk(BZ, BYY, 1);
-  dim3 grd((p.nz + BZ - 1) / BZ, (p.ny + BYY - 1) / BYY, p.nx);
+  const dim3 blk = block3(p.ny, p.nz), grd = grid3(blk, p.nx, p.ny, p.nz);
   int S = mp.stage_steps > 0 ? mp.stage_steps : 1;
   int filled = 0, first = step0;
   const long long e_cells = (long long)(p.nx - 1) * p.ny * p.nz + (long long)p.nx * (p.ny - 1) * p.nz +
