@@ -202,9 +202,9 @@ int run_t(mt_batch* b, int step0, int k, hipStream_t s) {
   const TmBatchVar<T>* vars = reinterpret_cast<const TmBatchVar<T>*>(b->ws + b->L.vars);
   const int* pin = reinterpret_cast<const int*>(b->ws + b->L.pre_in);
   const int* pring = reinterpret_cast<const int*>(b->ws + b->L.pre_ring);
+  LaunchSteps steps(k, S, b->NS);
   while (done < k) {
-    int nsub = std::min(b->NS, k - done);
-    if (b->max_mons) nsub = std::min(nsub, S - slot);
+    const int nsub = steps.next();
     rc = (b->dtype == MT_F64)
              ? tm_batch_dispatch_f64(b->variant, reinterpret_cast<const TmBatchVar<double>*>(vars), pin, pring,
                                      b->nvar, b->n_in, b->n_ring, b->grid_in, b->grid_ring, nsub, cur,

@@ -662,9 +662,9 @@ int tm_run_tiled(const mt_tm2d* d, const mt_source2d* src, const double* coef, c
   const int NS = tiled_variant_steps(d->variant, d->dtype);
   const int S = mp.n_mons ? mp.stage_steps : k;
   int done = 0, slot = 0, first = step0, cur = 0, rc;
+  LaunchSteps steps(k, S, NS);
   while (done < k) {
-    int nsub = std::min(NS, k - done);
-    if (mp.n_mons) nsub = std::min(nsub, S - slot);
+    const int nsub = steps.next();
     T** in = cur ? B : A;
     T** out = cur ? A : B;
     p.Ez = in[0], p.Dz = in[1], p.Hx = in[2], p.Hy = in[3];
@@ -725,9 +725,9 @@ int te_run_tiled(const mt_te2d* d, const mt_source2d* src, const double* coef, c
   const int NS = tiled_variant_steps(d->variant, d->dtype);
   const int S = mp.n_mons ? mp.stage_steps : k;
   int done = 0, slot = 0, first = step0, cur = 0, rc;
+  LaunchSteps steps(k, S, NS);
   while (done < k) {
-    int nsub = std::min(NS, k - done);
-    if (mp.n_mons) nsub = std::min(nsub, S - slot);
+    const int nsub = steps.next();
     T** in = cur ? B : A;
     T** out = cur ? A : B;
     p.Hz = in[0], p.Dx = in[1], p.Dy = in[2], p.pEyx = in[3], p.pExy = in[4], p.pHzy = in[5], p.pHzx = in[6];
