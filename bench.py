@@ -465,36 +465,38 @@ def bench_c4(args):
         "roofline": roof, "adjoint_roofline": adj_roof}), flush=True)
 
 
-def _gemm_roofline(net, batch=64, reps=5):
-    """Roofline of the surrogate's GEMM kernel over every GEMM of `reps`
-    training passes (forward + backward) at `batch`: FLOPs and algorithmic
-    bytes (BF16 operands read once, FP32 result written, and read when
-    accumulated into) divided by the summed duration of those launches (HIP
-    events around each launch on its stream).  The FNO's products are thin
-    (reductions of 64-256 over 16384-wide activations, or 16384-deep over
-    256 outputs), so the bound is whichever of the MFMA and HBM fractions is
-    higher; both are reported."""
-    from meep_torch_amd.surrogate import _nn
+def _operator_roofline(net, batch=64, reps=5):
+    """Roofline of one training pass of the surrogate (forward + backward) at
+    `batch`: FLOPs of its products and algorithmic bytes of the passes over
+    the (batch, channels, points) activations (each pass's BF16 operands read
+    and results written once, the FP32 pre-activations written and read once)
+    divided by the pass's duration (HIP events on its stream, every launch of
+    the pass included).  The products are thin (a side of 64-320), so the
+    bound is whichever of the MFMA and HBM fractions is higher; both are
+    reported."""
     rho = torch.rand(batch, net.n, net.n, device="cuda")
     dout = torch.randn(batch, net.n_out, device="cuda")
     net.forward(rho)
     net.backward(dout)
     torch.cuda.synchronize()
-    _nn.PROFILE = []
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    ev[0].record()
     for _ in range(reps):
         net.forward(rho)
         net.backward(dout)
+    ev[1].record()
     torch.cuda.synchronize()
-    rec, _nn.PROFILE = _nn.PROFILE, None
-    flops = sum(r[0] for r in rec)
-    nbytes = sum(r[1] for r in rec)
-    sec = sum(a.elapsed_time(b) for _, _, a, b in rec) * 1e-3
+    sec = ev[0].elapsed_time(ev[1]) * 1e-3 / reps
+    B, C, P, Mo, H, L = batch, net.C, net.P, net.Mo, net.H, net.L
+    dft, mix, point, head = 4 * B * P * C * Mo, 2 * B * Mo * (2 * C) ** 2, 2 * B * P * C * C, 2 * B * P * C * H
+    flops = L * (2 * dft + mix + point) + head + L * (2 * dft + 2 * mix + 2 * point) + 2 * head
+    act = B * C * P
+    nbytes = act * ((2 + 6 * L + 4 * (L - 1) + 2) + (4 + 8 * L + 4 * (L - 1) + 4))
     tf, gbs = flops / sec / 1e12, nbytes / sec / 1e9
     f_m, f_h = tf / 2500.0, gbs / HBM_PEAK_GBS
-    common = {"traffic": None, "kernel": f"gemm_kernel (BF16 MFMA, FP32 acc), all GEMMs of a B={batch} training pass",
-              "gemm_launches": len(rec) // reps, "gemm_flops_per_pass": flops / reps,
-              "gemm_alg_bytes_per_pass": nbytes / reps, "mfma_tflops": tf, "mfma_frac": f_m, "hbm_gbs": gbs,
-              "hbm_frac": f_h}
+    common = {"traffic": None, "kernel": f"spectral operator passes (BF16 MFMA, FP32 acc), one B={batch} training pass",
+              "flops_per_pass": flops, "alg_bytes_per_pass": nbytes, "mfma_tflops": tf, "mfma_frac": f_m,
+              "hbm_gbs": gbs, "hbm_frac": f_h}
     if f_h > f_m:
         return {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": f_h, **common}
     return {"bound": "mfma", "achieved": tf, "peak": 2500.0, "unit": "TFLOP/s", "frac": f_m, **common}
@@ -509,8 +511,8 @@ def bench_c5(args):
     net, data, hist = build_surrogate(pb, n_train=args.c5_solves, n_val=512, epochs=args.c5_epochs, log=log)
     torch.cuda.synchronize()
     setup_s = time.perf_counter() - t0
-    roof = _gemm_roofline(net)
-    log(f"[bench] c5 GEMM roofline: {roof['mfma_tflops']:.1f} TFLOP/s ({100 * roof['mfma_frac']:.1f}% of BF16 dense), "
+    roof = _operator_roofline(net)
+    log(f"[bench] c5 operator roofline: {roof['mfma_tflops']:.1f} TFLOP/s ({100 * roof['mfma_frac']:.1f}% of BF16 dense), "
         f"{roof['hbm_gbs']:.0f} GB/s of algorithmic bytes ({100 * roof['hbm_frac']:.1f}% of HBM): {roof['bound']}-bound")
     theta0 = D.start_design(pb)
     n_train = args.c5_solves
