@@ -232,25 +232,23 @@ class BatchedTM:
 
     def _forward_body(self):
         h, _ = self._plan(False)
-        for V in self.var:
-            for t in V["state"].values():
-                t.zero_()
-            for a in V["acc"]:
-                a.zero_()
+        # the copies and clears of every variant's fields in few launches: one
+        # each took 2.9 us, a tenth of a ten-variant gradient
+        state = [V["state"][f] for V in self.var for f in FIELDS]
+        chunk = [a for V in self.var for a in V["chunk_acc"]]
+        acc = [a for V in self.var for a in V["acc"]]
+        torch._foreach_zero_([t for V in self.var for t in V["state"].values()] + acc)
         step0, ci = 0, 0
         while step0 < self.n_steps:
             k = min(self.K, self.n_steps - step0)
-            for V in self.var:
-                if self.adjoint:
-                    for f in FIELDS:
-                        V["ckpt"][ci][f].copy_(V["state"][f])
-                for a in V["chunk_acc"]:
-                    a.zero_()
+            if self.adjoint:
+                torch._foreach_copy_([V["ckpt"][ci][f] for V in self.var for f in FIELDS], state)
+            if chunk:
+                torch._foreach_zero_(chunk)
             rc = self.L.mt_tm2d_batch_run(h, step0, k, E.stream_handle())
             E.check(rc, "mt_tm2d_batch_run")
-            for V in self.var:
-                for a, ca in zip(V["acc"], V["chunk_acc"]):
-                    a.add_(ca)
+            if chunk:
+                torch._foreach_add_(acc, chunk)
             step0 += k
             ci += 1
 
@@ -357,17 +355,13 @@ class BatchedTM:
     def _gradient_body(self):
         adj = self._adj
         h = adj["h"]
-        for P in adj["per"]:
-            for t in P["A"].values():
-                t.zero_()
-            P["g"].zero_()
+        torch._foreach_zero_([t for P in adj["per"] for t in (*P["A"].values(), P["g"])])
+        state = [V["state"][f] for V in self.var for f in FIELDS]
         nck = len(self.var[0]["ckpt"])
         for ci in reversed(range(nck)):
             step0 = ci * self.K
             k = min(self.K, self.n_steps - step0)
-            for V in self.var:
-                for f in FIELDS:
-                    V["state"][f].copy_(V["ckpt"][ci][f])
+            torch._foreach_copy_(state, [V["ckpt"][ci][f] for V in self.var for f in FIELDS])
             rc = self.L.mt_tm2d_batch_run(h, step0, k, E.stream_handle())
             E.check(rc, "mt_tm2d_batch_run (recompute)")
             rc = self.L.mt_tm2d_batch_adjoint_sweep(h, step0, k, E.stream_handle())
