@@ -451,6 +451,7 @@ extern "C" mt_batch* mt_tm2d_batch_create(const mt_tm2d_batch_item* items, int n
     return nullptr;
   }
   int max_mons = 0;
+  bool avg_d = false;
   for (int v = 0; v < nvar; ++v) {
     const mt_tm2d& d = items[v].prob;
     if (d.dtype != dtype) {
@@ -495,13 +496,14 @@ extern "C" mt_batch* mt_tm2d_batch_create(const mt_tm2d_batch_item* items, int n
       if (monitors_validate(mp)) return nullptr;
     }
     max_mons = std::max(max_mons, items[v].n_mons);
+    avg_d = avg_d || taps_avg_d(items[v].mons, items[v].n_mons);
   }
   mt_batch* b = new mt_batch();
   b->nvar = nvar;
   b->dtype = dtype;
-  b->variant = variant;
+  b->variant = avg_d ? kAvgVariant : variant;
   b->S = stage_steps > 0 ? stage_steps : 1;
-  b->NS = tiled_variant_steps(variant, dtype);
+  b->NS = tiled_variant_steps(b->variant, dtype);
   b->max_mons = max_mons;
   b->ws = static_cast<char*>(dev_ws);
   b->L = dtype == MT_F64 ? layout<double>(nvar) : layout<float>(nvar);

@@ -356,6 +356,13 @@ static int sample_t(const MonitorPlan& mp, int slot, int t_rel, hipStream_t s) {
   return check_launch("monitor gather");
 }
 
+bool taps_avg_d(const mt_monitor* mons, int n) {
+  for (int i = 0; i < n; ++i)
+    for (int q = 0; q < mons[i].n_terms; ++q)
+      if (mons[i].term[q].field >= 3 && mons[i].term[q].b && mons[i].term[q].line <= 2) return true;
+  return false;
+}
+
 bool build_taps(const MonitorPlan& mp, int slot0, int t_rel0, int esz, TapSet* out) {
   out->n = 0;
   char* base = static_cast<char*>(mp.stage);
@@ -366,7 +373,6 @@ bool build_taps(const MonitorPlan& mp, int slot0, int t_rel0, int esz, TapSet* o
     for (int q = 0; q < m.n_terms; ++q) {
       const mt_dft_term& tm = m.term[q];
       if (tm.line < 1 || tm.line > 4 || out->n >= kMaxTaps) return false;
-      if (tm.field >= 3 && tm.b) return false;  // D values are not averaged in a tile
       Tap& t = out->t[out->n++];
       t.field = tm.field;
       t.line = tm.line;

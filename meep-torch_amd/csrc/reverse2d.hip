@@ -508,7 +508,7 @@ bool rev_terms_ok(const mt_monitor* mons, int n) {
   for (int i = 0; i < n; ++i)
     for (int q = 0; q < mons[i].n_terms; ++q) {
       const mt_dft_term& t = mons[i].term[q];
-      if (t.line < 1 || t.line > 4 || t.field < 0 || t.field > 3 || (t.b && (t.line > 2 || t.field > 2))) return false;
+      if (t.line < 1 || t.line > 4 || t.field < 0 || t.field > 3 || (t.b && t.line > 2)) return false;
     }
   return true;
 }

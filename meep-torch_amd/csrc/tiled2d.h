@@ -90,6 +90,10 @@ int tm_batch_dispatch_f64(int variant, const TmBatchVar<double>* vars, const int
                           int t0, int slot_base, int tape_s0, hipStream_t s);
 TileMap tiled_map(int variant, int dtype, int nx, int ny, int in_i0, int in_i1, int in_j0, int in_j1);
 int tiled_variant_count();
+// The tile form for runs in which some monitor term averages D (taps_avg_d),
+// beyond the variants that callers choose from.
+constexpr int kAvgVariant = 1000;
+bool taps_avg_d(const mt_monitor* mons, int n);
 int tiled_variant_steps(int variant, int dtype);
 
 // Steps of each launch of a run of k steps: blocks of S steps (the monitors'

@@ -62,16 +62,17 @@ __device__ __forceinline__ bool taps_touch(const TapSet& taps, int I0, int J0, i
 }
 
 // Write this tile's share of every monitor term after sub-step `s`.
-// FIELD(id, li, lj) returns the LDS value of field `id` at local cell; terms
-// of fields from D0 up (D, which only the owning thread's registers hold)
-// are left to write_taps_own.
-template <typename T, int RX, int RY, int D0, typename F>
+// FIELD(id, li, lj) returns the LDS value of field `id` at local cell, for the
+// terms of fields F0 to F1 - 1.  D (ids from 3 up) lives in the owning thread's
+// registers: its terms are left to write_taps_own, or D visits the LDS where
+// some term averages it (AVGD).
+template <typename T, int RX, int RY, int F0, int F1, typename F>
 __device__ void write_taps(const TapSet& taps, int s, int I0, int J0, int TXo, int TYo, int a0, int b0,
                            F field, int slot_base) {
   const int tid = threadIdx.x;
   for (int q = 0; q < taps.n; ++q) {
     const Tap& t = taps.t[q];
-    if (t.field >= D0) continue;
+    if ((F0 > 0 && t.field < F0) || t.field >= F1) continue;
     T* out = static_cast<T*>(t.out) + (long long)(t.slot0 + slot_base + s) * t.slot_stride;
     if (t.line == 1) {  // row: fixed i = fix, j = lo + e
       if (t.fix < I0 || t.fix >= I0 + TXo) continue;
@@ -108,7 +109,7 @@ __device__ void write_taps(const TapSet& taps, int s, int I0, int J0, int TXo, i
 }
 
 // The terms of one D field (id `field`): an owned cell (i, j) with value v
-// writes itself (D terms are never averaged; build_taps sees to it).
+// writes itself (no term averages D; else the AVGD form runs).
 template <typename T>
 __device__ __forceinline__ void write_taps_own(const TapSet& taps, int s, int field, int i, int j, T v,
                                                int slot_base) {
@@ -147,7 +148,7 @@ __device__ __forceinline__ T box_w(const mt_source2d& s, int i, int j) {
 }
 
 // ------------------------------------------------------------------- TE
-template <typename T, int TX, int TY, int NS, int MAXB, bool PML>
+template <typename T, int TX, int TY, int NS, int MAXB, bool PML, bool AVGD>
 __device__ __forceinline__ void te_tile(const TeTiled<T>& p, const TapSet& taps, int nsub, int write_e, int tr,
                                         int tc, T* sm) {
   using S = Shape<TX, TY, NS, MAXB>;
@@ -291,14 +292,19 @@ __device__ __forceinline__ void te_tile(const TeTiled<T>& p, const TapSet& taps,
     }
     __syncthreads();
     if (tap_tile) {
-      write_taps<T, RX, RY, 3>(
-          taps, s, I0, J0, TX, TY, a0, b0,
-          [&](int f, int li, int lj) -> T {
-            int c = li * RY + lj;
-            return f == 0 ? sHz[c] : f == 1 ? sEx[c] : sEy[c];
-          },
-          0);
-      if (tap_d) {
+      auto field = [&](int f, int li, int lj) -> T {
+        int c = li * RY + lj;
+        return f == 0 ? sHz[c] : f == 1 || (AVGD && f == 3) ? sEx[c] : sEy[c];
+      };
+      write_taps<T, RX, RY, 0, 3>(taps, s, I0, J0, TX, TY, a0, b0, field, 0);
+      if (AVGD && tap_d) {   // D takes the place of E, which the next D half writes before it is read
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < PER; ++u)
+          if (ok(u)) sEx[tid + u * STR] = vDx[u], sEy[tid + u * STR] = vDy[u];
+        __syncthreads();
+        write_taps<T, RX, RY, 3, 5>(taps, s, I0, J0, TX, TY, a0, b0, field, 0);
+      } else if (tap_d) {
 #pragma unroll
         for (int u = 0; u < PER; ++u) {
           const int i = i0 + u * ROWS;
@@ -339,7 +345,7 @@ __device__ __forceinline__ void te_tile(const TeTiled<T>& p, const TapSet& taps,
 }
 
 // ------------------------------------------------------------------- TM
-template <typename T, int TX, int TY, int NS, int MAXB, bool PML>
+template <typename T, int TX, int TY, int NS, int MAXB, bool PML, bool AVGD = false>
 __device__ __forceinline__ void tm_tile(const TmTiled<T>& p, const TapSet& taps, int nsub, int tape_s0, int tr,
                                         int tc, int slot_base, int coef_t0, T* sm) {
   using S = Shape<TX, TY, NS, MAXB>;
@@ -506,14 +512,19 @@ __device__ __forceinline__ void tm_tile(const TmTiled<T>& p, const TapSet& taps,
         if (own(u)) tape[(long long)(tape_s0 + s) * nx * ny + (long long)(i0 + u * ROWS) * ny + j] = vEz[u];
     }
     if (tap_tile) {
-      write_taps<T, RX, RY, 3>(
-          taps, s, I0, J0, TX, TY, a0, b0,
-          [&](int f, int li, int lj) -> T {
-            int c = li * RY + lj;
-            return f == 0 ? sEz[c] : f == 1 ? sHx[c] : sHy[c];
-          },
-          slot_base);
-      if (tap_d) {
+      auto field = [&](int f, int li, int lj) -> T {
+        int c = li * RY + lj;
+        return f == 0 ? sEz[c] : f == 1 || (AVGD && f == 3) ? sHx[c] : sHy[c];
+      };
+      write_taps<T, RX, RY, 0, 3>(taps, s, I0, J0, TX, TY, a0, b0, field, slot_base);
+      if (AVGD && tap_d) {   // Dz takes the place of Hx, which the next B half writes before it is read
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < PER; ++u)
+          if (ok(u)) sHx[tid + u * STR] = vDz[u];
+        __syncthreads();
+        write_taps<T, RX, RY, 3, 4>(taps, s, I0, J0, TX, TY, a0, b0, field, slot_base);
+      } else if (tap_d) {
 #pragma unroll
         for (int u = 0; u < PER; ++u)
           if (own(u)) write_taps_own<T>(taps, s, 3, i0 + u * ROWS, j, vDz[u], slot_base);
@@ -559,28 +570,28 @@ constexpr int lds_elems() {
   return 3 * S::RC + (PML ? 4 * S::RX : 0);
 }
 
-template <typename T, int TX, int TY, int NS, int MAXB, int MODE>
+template <typename T, int TX, int TY, int NS, int MAXB, int MODE, bool AVGD>
 __global__ __launch_bounds__((Shape<TX, TY, NS, MAXB>::BLK)) void te_tiled(TeTiled<T> p, TapSet taps, int nsub,
                                                                           int write_e) {
   __shared__ T sm[lds_elems<T, TX, TY, NS, MAXB, MODE != kInterior>()];
   int tr, tc;
   const bool pml = pick_tile<MODE>(p.map, &tr, &tc);
   if (MODE == kRing || (MODE == kAll && pml))
-    te_tile<T, TX, TY, NS, MAXB, true>(p, taps, nsub, write_e, tr, tc, sm);
+    te_tile<T, TX, TY, NS, MAXB, true, AVGD>(p, taps, nsub, write_e, tr, tc, sm);
   else
-    te_tile<T, TX, TY, NS, MAXB, false>(p, taps, nsub, write_e, tr, tc, sm);
+    te_tile<T, TX, TY, NS, MAXB, false, AVGD>(p, taps, nsub, write_e, tr, tc, sm);
 }
 
-template <typename T, int TX, int TY, int NS, int MODE>
+template <typename T, int TX, int TY, int NS, int MODE, bool AVGD>
 __global__ __launch_bounds__((Shape<TX, TY, NS, kMaxTm>::BLK)) void tm_tiled(TmTiled<T> p, TapSet taps, int nsub,
                                                                            int tape_s0) {
   __shared__ T sm[lds_elems<T, TX, TY, NS, kMaxTm, MODE != kInterior>()];
   int tr, tc;
   const bool pml = pick_tile<MODE>(p.map, &tr, &tc);
   if (MODE == kRing || (MODE == kAll && pml))
-    tm_tile<T, TX, TY, NS, kMaxTm, true>(p, taps, nsub, tape_s0, tr, tc, 0, 0, sm);
+    tm_tile<T, TX, TY, NS, kMaxTm, true, AVGD>(p, taps, nsub, tape_s0, tr, tc, 0, 0, sm);
   else
-    tm_tile<T, TX, TY, NS, kMaxTm, false>(p, taps, nsub, tape_s0, tr, tc, 0, 0, sm);
+    tm_tile<T, TX, TY, NS, kMaxTm, false, AVGD>(p, taps, nsub, tape_s0, tr, tc, 0, 0, sm);
 }
 
 // FP32 interior tiles held to 64 VGPRs (eight waves per SIMD): two
@@ -602,7 +613,7 @@ tm_tiled_in2(TmTiled<T> p, TapSet taps, int nsub, int tape_s0) {
 // (both ping-pong orientations), taps and tile maps live in device memory, so
 // the launch depends only on scalars and can be captured in a graph and
 // replayed.
-template <typename T, int TX, int TY, int NS, int MODE>
+template <typename T, int TX, int TY, int NS, int MODE, bool AVGD>
 __device__ __forceinline__ void tm_batch_body(const TmBatchVar<T>* vars, const int* pre_in, const int* pre_ring,
                                               int nvar, int nsub, int parity, int t0, int slot_base, int tape_s0,
                                               T* sm) {
@@ -629,20 +640,20 @@ __device__ __forceinline__ void tm_batch_body(const TmBatchVar<T>* vars, const i
     int tr, tc;
     tile_linear(ring, p.map, it - prefix[lo], &tr, &tc);
     if (MODE == kRing || (MODE == kAll && ring))
-      tm_tile<T, TX, TY, NS, kMaxTm, true>(p, V.taps, nsub, tape_s0, tr, tc, slot_base, t0, sm);
+      tm_tile<T, TX, TY, NS, kMaxTm, true, AVGD>(p, V.taps, nsub, tape_s0, tr, tc, slot_base, t0, sm);
     else
-      tm_tile<T, TX, TY, NS, kMaxTm, false>(p, V.taps, nsub, tape_s0, tr, tc, slot_base, t0, sm);
+      tm_tile<T, TX, TY, NS, kMaxTm, false, AVGD>(p, V.taps, nsub, tape_s0, tr, tc, slot_base, t0, sm);
     __syncthreads();
   }
 }
 
-template <typename T, int TX, int TY, int NS, int MODE>
+template <typename T, int TX, int TY, int NS, int MODE, bool AVGD>
 __global__ __launch_bounds__((Shape<TX, TY, NS, kMaxTm>::BLK)) void tm_batch(const TmBatchVar<T>* vars,
                                                                            const int* pre_in, const int* pre_ring,
                                                                            int nvar, int nsub, int parity, int t0,
                                                                            int slot_base, int tape_s0) {
   __shared__ T sm[lds_elems<T, TX, TY, NS, kMaxTm, MODE != kInterior>()];
-  tm_batch_body<T, TX, TY, NS, MODE>(vars, pre_in, pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0, sm);
+  tm_batch_body<T, TX, TY, NS, MODE, AVGD>(vars, pre_in, pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0, sm);
 }
 
 // the interior form held to 64 VGPRs, as tm_tiled_in2
@@ -651,7 +662,7 @@ __global__ __launch_bounds__((Shape<TX, TY, NS, kMaxTm>::BLK)) __attribute__((am
 tm_batch_in2(const TmBatchVar<T>* vars, const int* pre_in, const int* pre_ring, int nvar, int nsub, int parity,
              int t0, int slot_base, int tape_s0) {
   __shared__ T sm[lds_elems<T, TX, TY, NS, kMaxTm, false>()];
-  tm_batch_body<T, TX, TY, NS, kInterior>(vars, pre_in, pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0, sm);
+  tm_batch_body<T, TX, TY, NS, kInterior, false>(vars, pre_in, pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0, sm);
 }
 
 }  // namespace
@@ -684,44 +695,44 @@ void launch_tiles(const TileMap& m, KA kall, K1 kin, K2 kpml, hipStream_t s, lon
   if (n_ring) kpml(dim3(n_ring));
 }
 
-template <typename T, int TX, int TY, int NS>
+template <typename T, int TX, int TY, int NS, bool AVGD = false>
 int launch_te_tiled(TeTiled<T> p, const TapSet& taps, int nsub, int write_e, hipStream_t s) {
   constexpr int MI = te_max<TX, TY, NS>(false), MR = te_max<TX, TY, NS>(true);
   p.map = make_map<TX, TY, NS>(p.nx, p.ny, p.in_i0, p.in_i1, p.in_j0, p.in_j1);
   launch_tiles(
       p.map,
       [&](dim3 g) {
-        hipLaunchKernelGGL((te_tiled<T, TX, TY, NS, MR, kAll>), g, dim3(Shape<TX, TY, NS, MR>::BLK), 0, s, p, taps, nsub, write_e);
+        hipLaunchKernelGGL((te_tiled<T, TX, TY, NS, MR, kAll, AVGD>), g, dim3(Shape<TX, TY, NS, MR>::BLK), 0, s, p, taps, nsub, write_e);
       },
       [&](dim3 g) {
-        hipLaunchKernelGGL((te_tiled<T, TX, TY, NS, MI, kInterior>), g, dim3(Shape<TX, TY, NS, MI>::BLK), 0, s, p, taps, nsub, write_e);
+        hipLaunchKernelGGL((te_tiled<T, TX, TY, NS, MI, kInterior, AVGD>), g, dim3(Shape<TX, TY, NS, MI>::BLK), 0, s, p, taps, nsub, write_e);
       },
       [&](dim3 g) {
-        hipLaunchKernelGGL((te_tiled<T, TX, TY, NS, MR, kRing>), g, dim3(Shape<TX, TY, NS, MR>::BLK), 0, s, p, taps, nsub, write_e);
+        hipLaunchKernelGGL((te_tiled<T, TX, TY, NS, MR, kRing, AVGD>), g, dim3(Shape<TX, TY, NS, MR>::BLK), 0, s, p, taps, nsub, write_e);
       },
       s, (long long)TX * TY, nsub);
   return check_launch("te2d tiled step");
 }
 
-template <typename T, int TX, int TY, int NS>
+template <typename T, int TX, int TY, int NS, bool AVGD = false>
 int launch_tm_tiled(TmTiled<T> p, const TapSet& taps, int nsub, int tape_s0, hipStream_t s) {
   constexpr int BLK = Shape<TX, TY, NS, kMaxTm>::BLK;
   p.map = make_map<TX, TY, NS>(p.nx, p.ny, p.in_i0, p.in_i1, p.in_j0, p.in_j1);
   launch_tiles(
       p.map,
-      [&](dim3 g) { hipLaunchKernelGGL((tm_tiled<T, TX, TY, NS, kAll>), g, dim3(BLK), 0, s, p, taps, nsub, tape_s0); },
+      [&](dim3 g) { hipLaunchKernelGGL((tm_tiled<T, TX, TY, NS, kAll, AVGD>), g, dim3(BLK), 0, s, p, taps, nsub, tape_s0); },
       [&](dim3 g) {
-        if constexpr (sizeof(T) == 4)
+        if constexpr (sizeof(T) == 4 && !AVGD)
           hipLaunchKernelGGL((tm_tiled_in2<T, TX, TY, NS>), g, dim3(BLK), 0, s, p, taps, nsub, tape_s0);
         else
-          hipLaunchKernelGGL((tm_tiled<T, TX, TY, NS, kInterior>), g, dim3(BLK), 0, s, p, taps, nsub, tape_s0);
+          hipLaunchKernelGGL((tm_tiled<T, TX, TY, NS, kInterior, AVGD>), g, dim3(BLK), 0, s, p, taps, nsub, tape_s0);
       },
-      [&](dim3 g) { hipLaunchKernelGGL((tm_tiled<T, TX, TY, NS, kRing>), g, dim3(BLK), 0, s, p, taps, nsub, tape_s0); },
+      [&](dim3 g) { hipLaunchKernelGGL((tm_tiled<T, TX, TY, NS, kRing, AVGD>), g, dim3(BLK), 0, s, p, taps, nsub, tape_s0); },
       s, (long long)TX * TY, nsub);
   return check_launch("tm2d tiled step");
 }
 
-template <typename T, int TX, int TY, int NS>
+template <typename T, int TX, int TY, int NS, bool AVGD = false>
 int launch_tm_batch(const TmBatchVar<T>* vars, const int* pre_in, const int* pre_ring, int nvar, int n_in,
                     int n_ring, int grid_in, int grid_ring, int nsub, int parity, int t0, int slot_base,
                     int tape_s0, hipStream_t s) {
@@ -729,23 +740,23 @@ int launch_tm_batch(const TmBatchVar<T>* vars, const int* pre_in, const int* pre
   const int n = n_in + n_ring;
   if (n <= kOneRound && n_in && n_ring) {
     timing_begin(s);
-    hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, kAll>), dim3(n), dim3(BLK), 0, s, vars, pre_in, pre_ring, nvar,
+    hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, kAll, AVGD>), dim3(n), dim3(BLK), 0, s, vars, pre_in, pre_ring, nvar,
                        nsub, parity, t0, slot_base, tape_s0);
     timing_end(s, (long long)n * TX * TY * nsub);
     return check_launch("tm2d batched step");
   }
   if (n_in) {
     timing_begin(s);
-    if constexpr (sizeof(T) == 4)
+    if constexpr (sizeof(T) == 4 && !AVGD)
       hipLaunchKernelGGL((tm_batch_in2<T, TX, TY, NS>), dim3(std::min(n_in, grid_in)), dim3(BLK), 0, s, vars,
                          pre_in, pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0);
     else
-      hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, kInterior>), dim3(std::min(n_in, grid_in)), dim3(BLK), 0, s, vars,
+      hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, kInterior, AVGD>), dim3(std::min(n_in, grid_in)), dim3(BLK), 0, s, vars,
                          pre_in, pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0);
     timing_end(s, (long long)n_in * TX * TY * nsub);
   }
   if (n_ring)
-    hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, kRing>), dim3(std::min(n_ring, grid_ring)), dim3(BLK), 0, s, vars,
+    hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, kRing, AVGD>), dim3(std::min(n_ring, grid_ring)), dim3(BLK), 0, s, vars,
                        pre_in, pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0);
   return check_launch("tm2d batched step");
 }
@@ -772,6 +783,11 @@ TileMap map_for(int nx, int ny, int in_i0, int in_i1, int in_j0, int in_j1) {
   X(T, 8, 64, 1) X(T, 8, 64, 2) X(T, 8, 64, 4) X(T, 16, 64, 1) X(T, 16, 64, 2) X(T, 16, 32, 2) X(T, 8, 128, 1) \
   X(T, 16, 16, 6) X(T, 8, 8, 8) X(T, 16, 32, 4)
 constexpr int kVariants = 10;
+// Runs with a term that averages D take this shape (kAvgVariant in the
+// dispatches) whatever variant was asked for: D visits the LDS for such terms,
+// and as a branch in every kernel that cost 2% of the TM cases and 6% of a batch of
+// ten variants.
+constexpr int kAvgShape = 1;
 static const int kVarF32[kVariants][3] = {{16, 64, 1}, {16, 64, 2}, {16, 64, 4}, {32, 64, 1}, {32, 64, 2},
                                           {32, 64, 4}, {8, 128, 2}, {16, 16, 7}, {8, 8, 8}, {16, 32, 4}};
 static const int kVarF64[kVariants][3] = {{8, 64, 1}, {8, 64, 2}, {8, 64, 4}, {16, 64, 1}, {16, 64, 2},
@@ -784,6 +800,7 @@ int te_tiled_dispatch_f32(int variant, const TeTiled<float>& p, const TapSet& ta
   if (variant == v++) return launch_te_tiled<T, A, B, C>(p, taps, nsub, write_e, s);
   MT_VARIANTS_F32(X, float)
 #undef X
+  if (variant == kAvgVariant) return launch_te_tiled<float, 16, 64, 2, true>(p, taps, nsub, write_e, s);
   return fail(MT_EINVAL, "unknown tiled variant");
 }
 
@@ -794,6 +811,7 @@ int te_tiled_dispatch_f64(int variant, const TeTiled<double>& p, const TapSet& t
   if (variant == v++) return launch_te_tiled<T, A, B, C>(p, taps, nsub, write_e, s);
   MT_VARIANTS_F64(X, double)
 #undef X
+  if (variant == kAvgVariant) return launch_te_tiled<double, 8, 64, 2, true>(p, taps, nsub, write_e, s);
   return fail(MT_EINVAL, "unknown tiled variant");
 }
 
@@ -804,6 +822,7 @@ int tm_tiled_dispatch_f32(int variant, const TmTiled<float>& p, const TapSet& ta
   if (variant == v++) return launch_tm_tiled<T, A, B, C>(p, taps, nsub, tape_s0, s);
   MT_VARIANTS_F32(X, float)
 #undef X
+  if (variant == kAvgVariant) return launch_tm_tiled<float, 16, 64, 2, true>(p, taps, nsub, tape_s0, s);
   return fail(MT_EINVAL, "unknown tiled variant");
 }
 
@@ -814,6 +833,7 @@ int tm_tiled_dispatch_f64(int variant, const TmTiled<double>& p, const TapSet& t
   if (variant == v++) return launch_tm_tiled<T, A, B, C>(p, taps, nsub, tape_s0, s);
   MT_VARIANTS_F64(X, double)
 #undef X
+  if (variant == kAvgVariant) return launch_tm_tiled<double, 8, 64, 2, true>(p, taps, nsub, tape_s0, s);
   return fail(MT_EINVAL, "unknown tiled variant");
 }
 
@@ -827,6 +847,9 @@ int tm_batch_dispatch_f32(int variant, const TmBatchVar<float>* vars, const int*
                                        nsub, parity, t0, slot_base, tape_s0, s);
   MT_VARIANTS_F32(X, float)
 #undef X
+  if (variant == kAvgVariant)
+    return launch_tm_batch<float, 16, 64, 2, true>(vars, pre_in, pre_ring, nvar, n_in, n_ring, grid_in, grid_ring, nsub,
+                                                parity, t0, slot_base, tape_s0, s);
   return fail(MT_EINVAL, "unknown tiled variant");
 }
 
@@ -840,10 +863,14 @@ int tm_batch_dispatch_f64(int variant, const TmBatchVar<double>* vars, const int
                                        nsub, parity, t0, slot_base, tape_s0, s);
   MT_VARIANTS_F64(X, double)
 #undef X
+  if (variant == kAvgVariant)
+    return launch_tm_batch<double, 8, 64, 2, true>(vars, pre_in, pre_ring, nvar, n_in, n_ring, grid_in, grid_ring, nsub,
+                                                parity, t0, slot_base, tape_s0, s);
   return fail(MT_EINVAL, "unknown tiled variant");
 }
 
 TileMap tiled_map(int variant, int dtype, int nx, int ny, int in_i0, int in_i1, int in_j0, int in_j1) {
+  if (variant == kAvgVariant) variant = kAvgShape;
   int v = 0;
 #define X(T, A, B, C) \
   if (variant == v++) return map_for<A, B, C>(nx, ny, in_i0, in_i1, in_j0, in_j1);
@@ -859,6 +886,7 @@ TileMap tiled_map(int variant, int dtype, int nx, int ny, int in_i0, int in_i1, 
 int tiled_variant_count() { return kVariants; }
 
 int tiled_variant_steps(int variant, int dtype) {
+  if (variant == kAvgVariant) variant = kAvgShape;
   if (variant < 0 || variant >= kVariants) return 0;
   return dtype == MT_F64 ? kVarF64[variant][2] : kVarF32[variant][2];
 }

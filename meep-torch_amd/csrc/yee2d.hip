@@ -659,7 +659,8 @@ int tm_run_tiled(const mt_tm2d* d, const mt_source2d* src, const double* coef, c
   p.hsrc[0] = d->hsrc[0];
   p.hsrc[1] = d->hsrc[1];
   const bool hsrc = d->hsrc[0].present || d->hsrc[1].present;
-  const int NS = tiled_variant_steps(d->variant, d->dtype);
+  const int variant = taps_avg_d(mp.mons, mp.n_mons) ? kAvgVariant : d->variant;
+  const int NS = tiled_variant_steps(variant, d->dtype);
   const int S = mp.n_mons ? mp.stage_steps : k;
   int done = 0, slot = 0, first = step0, cur = 0, rc;
   LaunchSteps steps(k, S, NS);
@@ -677,7 +678,7 @@ int tm_run_tiled(const mt_tm2d* d, const mt_source2d* src, const double* coef, c
     TapSet taps;
     taps.n = 0;
     if (mp.n_mons && !build_taps(mp, slot, done, sizeof(T), &taps)) return fail(MT_EINVAL, "tap build failed");
-    rc = P::tm(d->variant, p, taps, nsub, done, s);
+    rc = P::tm(variant, p, taps, nsub, done, s);
     if (rc) return rc;
     cur ^= 1;
     done += nsub;
@@ -722,7 +723,8 @@ int te_run_tiled(const mt_te2d* d, const mt_source2d* src, const double* coef, c
   p.Ex = static_cast<T*>(d->Ex);
   p.Ey = static_cast<T*>(d->Ey);
   if (src && src->present) p.src = *src;
-  const int NS = tiled_variant_steps(d->variant, d->dtype);
+  const int variant = taps_avg_d(mp.mons, mp.n_mons) ? kAvgVariant : d->variant;
+  const int NS = tiled_variant_steps(variant, d->dtype);
   const int S = mp.n_mons ? mp.stage_steps : k;
   int done = 0, slot = 0, first = step0, cur = 0, rc;
   LaunchSteps steps(k, S, NS);
@@ -738,7 +740,7 @@ int te_run_tiled(const mt_te2d* d, const mt_source2d* src, const double* coef, c
     TapSet taps;
     taps.n = 0;
     if (mp.n_mons && !build_taps(mp, slot, done, sizeof(T), &taps)) return fail(MT_EINVAL, "tap build failed");
-    rc = P::te(d->variant, p, taps, nsub, done + nsub == k ? 1 : 0, s);
+    rc = P::te(variant, p, taps, nsub, done + nsub == k ? 1 : 0, s);
     if (rc) return rc;
     cur ^= 1;
     done += nsub;
@@ -776,7 +778,7 @@ struct DispF64 {
 bool taps_ok(const MonitorPlan& mp) {
   for (int i = 0; i < mp.n_mons; ++i)
     for (int q = 0; q < mp.mons[i].n_terms; ++q)
-      if (mp.mons[i].term[q].line == 0 || (mp.mons[i].term[q].field >= 3 && mp.mons[i].term[q].b)) return false;
+      if (mp.mons[i].term[q].line == 0) return false;
   return true;
 }
 
