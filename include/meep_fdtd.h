@@ -402,16 +402,20 @@ int mt_tm2d_adjoint(const mt_tm2d* p, const mt_tm2d_adj* a, const void* tape,
 
 /* The same reverse sweep, temporally blocked: several reverse steps per launch
  * on overlapped tiles (p->variant: the forward's tile variant ids), for
- * problems without media and symmetry cuts.  a holds the cotangents on entry
+ * problems without media and symmetry cuts and monitors that
+ * mt_tm2d_adjoint_tiles_ok accepts (mt_tm2d_adjoint takes any).  a holds the cotangents on entry
  * and on return, b is a second set of the same shapes (its eps_grad and
- * scratch are not read; nor are a's gHy..gEy).  Every monitor term needs its
- * field position (mt_dft_term field, line, fix, lo); stage is a workspace of
+ * scratch are not read; nor are a's gHy..gEy).  stage is a workspace of
  * mt_stage_bytes(mons, n_mons, stage_steps, dtype) bytes into which the
  * monitor cotangents of stage_steps steps are evaluated at a time.  Same
  * results as mt_tm2d_adjoint. */
 int mt_tm2d_adjoint_tiled(const mt_tm2d* p, const mt_tm2d_adj* a, const mt_tm2d_adj* b, const void* tape,
                           const mt_monitor* mons, int n_mons, void* stage, long long stage_bytes, int stage_steps,
                           int step0, int k, void* stream);
+/* 1 if the tiled sweep takes these monitors: at most 32 terms together, each
+ * with its field position (mt_dft_term field, line, fix, lo), averages on
+ * lines only; else 0. */
+int mt_tm2d_adjoint_tiles_ok(const mt_monitor* mons, int n_mons);
 
 /* Adjoint state and scratch of one TE problem (same shapes as the forward
  * state; psi cotangents are tracked inside the CPML shells only). */

@@ -38,7 +38,7 @@ struct RevPart {
   int s_hi, nsub, lo, stage;
 };
 std::vector<RevPart> rev_schedule(int k, int S, int NS);
-// Every term has a field position the reverse tiles know (averages of lines only).
+// At most kMaxTaps terms, each with a field position the reverse tiles know (averages of lines only).
 bool rev_terms_ok(const mt_monitor* mons, int n);
 int rev_steps(int dtype, int variant);
 TileMap rev_map(int dtype, int variant, int nx, int ny, int i0, int i1, int j0, int j1);

@@ -505,8 +505,10 @@ struct RevBatchLaunch {
 }  // namespace
 
 bool rev_terms_ok(const mt_monitor* mons, int n) {
+  int taps = 0;
   for (int i = 0; i < n; ++i)
     for (int q = 0; q < mons[i].n_terms; ++q) {
+      if (++taps > kMaxTaps) return false;
       const mt_dft_term& t = mons[i].term[q];
       if (t.line < 1 || t.line > 4 || t.field < 0 || t.field > 3 || (t.b && t.line > 2)) return false;
     }
@@ -663,6 +665,10 @@ bool adj_complete(const mt_tm2d_adj* a) {
 }  // namespace mt
 
 using namespace mt;
+
+extern "C" int mt_tm2d_adjoint_tiles_ok(const mt_monitor* mons, int n_mons) {
+  return n_mons == 0 || (mons && n_mons > 0 && rev_terms_ok(mons, n_mons)) ? 1 : 0;
+}
 
 extern "C" int mt_tm2d_adjoint_tiled(const mt_tm2d* p, const mt_tm2d_adj* a, const mt_tm2d_adj* b, const void* tape,
                                      const mt_monitor* mons, int n_mons, void* stage, long long stage_bytes,

@@ -157,6 +157,8 @@ def lib():
     L.mt_tm2d_adjoint_tiled.restype = c_int
     L.mt_tm2d_adjoint_tiled.argtypes = [P(TM2D), P(TM2DAdj), P(TM2DAdj), c_void_p, P(Monitor), c_int, c_void_p,
                                         c_ll, c_int, c_int, c_int, c_void_p]
+    L.mt_tm2d_adjoint_tiles_ok.restype = c_int
+    L.mt_tm2d_adjoint_tiles_ok.argtypes = [P(Monitor), c_int]
     L.mt_te2d_adjoint.restype = c_int
     L.mt_te2d_adjoint.argtypes = [P(TE2D), P(TE2DAdj), c_void_p, P(Monitor), c_int, c_int, c_int,
                                   c_void_p]

@@ -172,17 +172,12 @@ class _TMRun(torch.autograd.Function):
             extra["c3"] = torch.zeros(cdet.c3.shape, dtype=dtype, device=device)
             if cdet.c3.shape[0]:
                 a.c3_grad = extra["c3"].data_ptr()
-        # without media and cuts, when every monitor term has a field position:
-        # several reverse steps per launch on tiles, between two cotangent sets
+        # without media and cuts, when the tiles take the monitors: several
+        # reverse steps per launch on tiles, between two cotangent sets
         tiled = not (kerr or cdet.d1 is not None or cdet.h1x is not None or cdet.c1.shape[0] or cdet.mc1x is not None
-                     or cdet.y_mirror_lo or cdet.x_mirror_lo) and \
-            all(len(t) > 3 and t[3] is not None for m in monitors for t in m.engine_terms(adj)[1])
-        if tiled:
-            d.variant = tune.tile_for(dtype, [(nx, ny)])
-            adj2 = {f: t.clone() for f, t in adj.items()}
-            a2 = E.TM2DAdj()
-            for f in names:
-                setattr(a2, "a" + f, adj2[f].data_ptr())
+                     or cdet.y_mirror_lo or cdet.x_mirror_lo)
+        d.variant = tune.tile_for(dtype, [(nx, ny)])
+        a2 = None
         for step0, k, st in reversed(ctx.ckpts):
             work = {f: t.clone() for f, t in st.items()}
             a.ez_init = st["Ez"].data_ptr()
@@ -190,7 +185,12 @@ class _TMRun(torch.autograd.Function):
             engine2d.run_chunk("tm", work, cdet, step0, k, plan, [], tape=tape)
             g_chunk = _chunk_cotangents(monitors, gacc, step0, k)
             arr, n_used, keep = _adj_monitors(adj, monitors, g_chunk, dtype, device)
-            if tiled:
+            if tiled and L.mt_tm2d_adjoint_tiles_ok(arr, n_used):
+                if a2 is None:   # the second set; its psi outside the shells is never written
+                    adj2 = {f: t.clone() for f, t in adj.items()}
+                    a2 = E.TM2DAdj()
+                    for f in names:
+                        setattr(a2, "a" + f, adj2[f].data_ptr())
                 S, stage, nbytes = engine2d.stage_alloc(L, arr, n_used, E.dtype_code(dtype), device)
                 rc = L.mt_tm2d_adjoint_tiled(ctypes.byref(d), ctypes.byref(a), ctypes.byref(a2), E.ptr(tape), arr,
                                              n_used, E.ptr(stage) if stage is not None else None, nbytes, S,
