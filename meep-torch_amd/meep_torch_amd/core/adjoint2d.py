@@ -174,9 +174,10 @@ class _TMRun(torch.autograd.Function):
                 a.c3_grad = extra["c3"].data_ptr()
         # without media and cuts, when the tiles take the monitors: several
         # reverse steps per launch on tiles, between two cotangent sets
-        tiled = not (kerr or cdet.d1 is not None or cdet.h1x is not None or cdet.c1.shape[0] or cdet.mc1x is not None
-                     or cdet.y_mirror_lo or cdet.x_mirror_lo)
-        d.variant = tune.tile_for(dtype, [(nx, ny)])
+        forced = tune.forced_variant()
+        tiled = forced != -1 and not (kerr or cdet.d1 is not None or cdet.h1x is not None or cdet.c1.shape[0]
+                                      or cdet.mc1x is not None or cdet.y_mirror_lo or cdet.x_mirror_lo)
+        d.variant = tune.tile_for(dtype, [(nx, ny)]) if forced is None else forced
         a2 = None
         for step0, k, st in reversed(ctx.ckpts):
             work = {f: t.clone() for f, t in st.items()}

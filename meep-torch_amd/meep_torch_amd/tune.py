@@ -7,7 +7,7 @@ shapes on scratch copies of the real state, sources and monitors, once per
 problem signature (mode, grid, dtype, monitor layout), and cache the faster
 for the rest of the process; `tune` times any set of variants, the two-pass
 per-half-step path (-1) included.  MEEP_TORCH_AMD_VARIANT=<v> forces a variant
-(-1 = two-pass)."""
+(-1 = two-pass), forward and in the TM reverse sweep (-1 = step by step)."""
 import os
 
 import torch
@@ -53,6 +53,12 @@ def tile_for(dtype, grids):
     return LADDER[dtype][-1] if v is None else v
 
 
+def forced_variant():
+    """MEEP_TORCH_AMD_VARIANT as a number, None when unset."""
+    env = os.environ.get("MEEP_TORCH_AMD_VARIANT")
+    return None if env is None else int(env)
+
+
 def _key(mode, fields, monitors):
     ref = fields["Ez"] if mode == "tm" else fields["Hz"]
     return (mode, tuple(ref.shape), ref.dtype, ref.device.index,
@@ -60,9 +66,9 @@ def _key(mode, fields, monitors):
 
 
 def variant_for(mode, fields, coeffs, plan, monitors, k):
-    env = os.environ.get("MEEP_TORCH_AMD_VARIANT")
-    if env is not None:
-        return int(env)
+    v = forced_variant()
+    if v is not None:
+        return v
     if k <= 4:
         return -1
     ref = fields["Ez"] if mode == "tm" else fields["Hz"]
