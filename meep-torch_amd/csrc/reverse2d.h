@@ -31,13 +31,6 @@ struct TmRevVar {
   TapSet taps;
 };
 
-// One launch of a sweep: steps s_hi, s_hi - 1, ... (nsub of them) of the
-// staging block that starts at step lo; stage > 0: fill the block's first
-// `stage` slots before the launch.
-struct RevPart {
-  int s_hi, nsub, lo, stage;
-};
-std::vector<RevPart> rev_schedule(int k, int S, int NS);
 // At most kMaxTaps terms, each with a field position the reverse tiles know (averages of lines only).
 bool rev_terms_ok(const mt_monitor* mons, int n);
 int rev_steps(int dtype, int variant);

@@ -314,9 +314,8 @@ __global__ __launch_bounds__((Shape<TX, TY, NS, kMaxRev>::BLK)) void tm_reverse_
   __shared__ T sm[rev_lds<T, TX, TY, NS, MODE != kInterior>()];
   const int n_ring = MODE == kInterior ? 0 : pre_ring[nvar];
   const int total = n_ring + (MODE == kRing ? 0 : pre_in[nvar]);
-  const int x = blockIdx.x & 7, nx8 = ((int)gridDim.x - x + 7) >> 3;
-  const int chunk = (total + 7) >> 3, end = min(total, (x + 1) * chunk);
-  for (int item = x * chunk + (int)(blockIdx.x >> 3); item < end; item += nx8) {
+  const XcdItems deal = xcd_items(blockIdx.x, gridDim.x, total);
+  for (int item = deal.first; item < deal.end; item += deal.stride) {
     const bool ring = MODE == kRing || (MODE == kAll && item < n_ring);
     const int* prefix = ring ? pre_ring : pre_in;
     const int it = ring ? item : item - n_ring;
@@ -488,15 +487,15 @@ struct RevBatchLaunch {
     constexpr int BLK = Shape<TX, TY, NS, kMaxRev>::BLK;
     const int n = n_in + n_ring;
     if (n <= kOneRound && n_in && n_ring) {
-      hipLaunchKernelGGL((tm_reverse_batch<T, TX, TY, NS, kAll>), dim3(n), dim3(BLK), 0, s, vars, pre_in, pre_ring,
-                         nvar, nsub, parity, s_hi, slot_hi);
+      hipLaunchKernelGGL((tm_reverse_batch<T, TX, TY, NS, kAll>), dim3(one_round_grid(n)), dim3(BLK), 0, s, vars, pre_in,
+                         pre_ring, nvar, nsub, parity, s_hi, slot_hi);
       return MT_OK;
     }
     if (n_in)
-      hipLaunchKernelGGL((tm_reverse_batch<T, TX, TY, NS, kInterior>), dim3(std::min(n_in, grid)), dim3(BLK), 0, s,
+      hipLaunchKernelGGL((tm_reverse_batch<T, TX, TY, NS, kInterior>), dim3(std::min(one_round_grid(n_in), grid)), dim3(BLK), 0, s,
                          vars, pre_in, pre_ring, nvar, nsub, parity, s_hi, slot_hi);
     if (n_ring)
-      hipLaunchKernelGGL((tm_reverse_batch<T, TX, TY, NS, kRing>), dim3(std::min(n_ring, grid)), dim3(BLK), 0, s,
+      hipLaunchKernelGGL((tm_reverse_batch<T, TX, TY, NS, kRing>), dim3(std::min(one_round_grid(n_ring), grid)), dim3(BLK), 0, s,
                          vars, pre_in, pre_ring, nvar, nsub, parity, s_hi, slot_hi);
     return MT_OK;
   }
@@ -524,34 +523,6 @@ TileMap rev_map(int dtype, int variant, int nx, int ny, int i0, int i1, int j0, 
   const MapOf f{nx, ny, i0, i1, j0, j1, &m};
   dtype == MT_F64 ? with_shape<double>(variant, f) : with_shape<float>(variant, f);
   return m;
-}
-
-// Launch lengths of a sweep over k steps in blocks of S staged steps: NS steps
-// each, an even number of launches when k > 1 (the sets alternate, so the
-// cotangents then end where they began).
-std::vector<RevPart> rev_schedule(int k, int S, int NS) {
-  std::vector<RevPart> v;
-  for (int hi = k - 1; hi >= 0;) {
-    const int lo = std::max(0, hi + 1 - S);
-    for (int s = hi; s >= lo;) {
-      const int n = std::min(NS, s - lo + 1);
-      v.push_back(RevPart{s, n, lo, s == hi ? hi - lo + 1 : 0});
-      s -= n;
-    }
-    hi = lo - 1;
-  }
-  if (v.size() % 2 && k > 1)
-    for (size_t q = 0; q < v.size(); ++q)
-      if (v[q].nsub > 1) {
-        RevPart b = v[q];
-        v[q].nsub = b.nsub / 2;
-        b.s_hi -= v[q].nsub;
-        b.nsub -= v[q].nsub;
-        b.stage = 0;
-        v.insert(v.begin() + q + 1, b);
-        break;
-      }
-  return v;
 }
 
 template <typename T>

@@ -2,9 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-
 #include "common.h"
+#include "schedule.h"
 
 namespace mt {
 
@@ -95,36 +94,6 @@ int tiled_variant_count();
 constexpr int kAvgVariant = 1000;
 bool taps_avg_d(const mt_monitor* mons, int n);
 int tiled_variant_steps(int variant, int dtype);
-
-// Steps of each launch of a run of k steps: blocks of S steps (the monitors'
-// staging ring; S = k without monitors), NS per launch, the first launch of
-// several steps cut in two where the number would be odd, so that a run ends
-// in the buffers it began in.  The copy back that an odd number needs moves
-// eight arrays per grid, about the bytes of a launch, in eight (or, batched,
-// eight per variant) dependent copies of 3 us or more; a launch of half the
-// steps costs little over half.
-// Ten variants of 200 to 900 cells a side, forward and gradient over 400
-// steps in segments of 100: 50.4 -> 49.2 ms; 100 x 60 in FP64, 400 steps: 1.58 -> 1.56.
-struct LaunchSteps {
-  int NS, S, left, slot = 0, rest = 0;
-  bool cut;
-  LaunchSteps(int k, int S_, int NS_) : NS(NS_), S(S_), left(k) {
-    const long long n = S > 0 ? (long long)(k / S) * ((S + NS - 1) / NS) + (k % S + NS - 1) / NS : 0;
-    cut = n % 2 != 0;
-  }
-  int next() {
-    int n = rest ? rest : std::min(NS, std::min(left, S - slot));
-    rest = 0;
-    if (cut && n > 1) {
-      rest = n / 2;
-      n -= rest;
-      cut = false;
-    }
-    left -= n;
-    slot = (slot + n) % S;
-    return n;
-  }
-};
 
 // Build the tap set of a tiled launch from the monitor plan; false if some
 // term has no semantic form (then the per-half-step path must be used).

@@ -619,13 +619,8 @@ __device__ __forceinline__ void tm_batch_body(const TmBatchVar<T>* vars, const i
                                               T* sm) {
   const int n_ring = MODE == kInterior ? 0 : pre_ring[nvar];
   const int total = n_ring + (MODE == kRing ? 0 : pre_in[nvar]);
-  // XCD-aware order: workgroups are dealt to the eight XCDs round robin, so
-  // the blocks of XCD x (blockIdx % 8 == x) share the contiguous item range
-  // [x * chunk, (x + 1) * chunk): neighbouring tiles, whose halos overlap,
-  // run on the same XCD (same L2) at about the same time
-  const int x = blockIdx.x & 7, nx8 = ((int)gridDim.x - x + 7) >> 3;
-  const int chunk = (total + 7) >> 3, end = min(total, (x + 1) * chunk);
-  for (int item = x * chunk + (int)(blockIdx.x >> 3); item < end; item += nx8) {
+  const XcdItems deal = xcd_items(blockIdx.x, gridDim.x, total);
+  for (int item = deal.first; item < deal.end; item += deal.stride) {
     const bool ring = MODE == kRing || (MODE == kAll && item < n_ring);
     const int* prefix = ring ? pre_ring : pre_in;
     const int it = ring ? item : item - n_ring;
@@ -740,23 +735,23 @@ int launch_tm_batch(const TmBatchVar<T>* vars, const int* pre_in, const int* pre
   const int n = n_in + n_ring;
   if (n <= kOneRound && n_in && n_ring) {
     timing_begin(s);
-    hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, kAll, AVGD>), dim3(n), dim3(BLK), 0, s, vars, pre_in, pre_ring, nvar,
-                       nsub, parity, t0, slot_base, tape_s0);
+    hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, kAll, AVGD>), dim3(one_round_grid(n)), dim3(BLK), 0, s, vars, pre_in,
+                       pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0);
     timing_end(s, (long long)n * TX * TY * nsub);
     return check_launch("tm2d batched step");
   }
   if (n_in) {
     timing_begin(s);
     if constexpr (sizeof(T) == 4 && !AVGD)
-      hipLaunchKernelGGL((tm_batch_in2<T, TX, TY, NS>), dim3(std::min(n_in, grid_in)), dim3(BLK), 0, s, vars,
+      hipLaunchKernelGGL((tm_batch_in2<T, TX, TY, NS>), dim3(std::min(one_round_grid(n_in), grid_in)), dim3(BLK), 0, s, vars,
                          pre_in, pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0);
     else
-      hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, kInterior, AVGD>), dim3(std::min(n_in, grid_in)), dim3(BLK), 0, s, vars,
+      hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, kInterior, AVGD>), dim3(std::min(one_round_grid(n_in), grid_in)), dim3(BLK), 0, s, vars,
                          pre_in, pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0);
     timing_end(s, (long long)n_in * TX * TY * nsub);
   }
   if (n_ring)
-    hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, kRing, AVGD>), dim3(std::min(n_ring, grid_ring)), dim3(BLK), 0, s, vars,
+    hipLaunchKernelGGL((tm_batch<T, TX, TY, NS, kRing, AVGD>), dim3(std::min(one_round_grid(n_ring), grid_ring)), dim3(BLK), 0, s, vars,
                        pre_in, pre_ring, nvar, nsub, parity, t0, slot_base, tape_s0);
   return check_launch("tm2d batched step");
 }
