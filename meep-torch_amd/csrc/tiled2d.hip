@@ -558,11 +558,16 @@ __device__ __forceinline__ void tm_tile(const TmTiled<T>& p, const TapSet& taps,
 // Threads per workgroup, at most.  TM tiles and CPML tiles take up to 1024
 // (few cells per thread: their launches are latency chains); TE interior
 // tiles of the large shapes take 512 (on 2048^2 that launch is
-// arithmetic-bound and 1024-thread tiles measured slower, 98 -> 123 us).
+// arithmetic-bound and 1024-thread tiles measured slower, 98 -> 123 us).  FP64
+// TE interior tiles take two cells per thread: with one, two blocks fill a CU
+// (8 x 64 x 2 tiles on 2048^2, per two steps: 175 -> 113 us), with three, 101
+// registers do (16 x 64 x 2: 101 -> 98 us, 8 x 64 x 4 no faster).
 constexpr int kMaxTm = 1024;
-template <int TX, int TY, int NS>
+template <typename T, int TX, int TY, int NS>
 constexpr int te_max(bool pml) {
-  return pml || (TX + 2 * NS + 1) * (TY + 2 * NS + 1) <= 1100 ? 1024 : 512;
+  if (pml) return 1024;
+  const int cells = (TX + 2 * NS + 1) * (TY + 2 * NS + 1);
+  return sizeof(T) == 8 ? (cells <= 1024 ? 512 : 1024) : (cells <= 1100 ? 1024 : 512);
 }
 template <typename T, int TX, int TY, int NS, int MAXB, bool PML>
 constexpr int lds_elems() {
@@ -692,7 +697,7 @@ void launch_tiles(const TileMap& m, KA kall, K1 kin, K2 kpml, hipStream_t s, lon
 
 template <typename T, int TX, int TY, int NS, bool AVGD = false>
 int launch_te_tiled(TeTiled<T> p, const TapSet& taps, int nsub, int write_e, hipStream_t s) {
-  constexpr int MI = te_max<TX, TY, NS>(false), MR = te_max<TX, TY, NS>(true);
+  constexpr int MI = te_max<T, TX, TY, NS>(false), MR = te_max<T, TX, TY, NS>(true);
   p.map = make_map<TX, TY, NS>(p.nx, p.ny, p.in_i0, p.in_i1, p.in_j0, p.in_j1);
   launch_tiles(
       p.map,

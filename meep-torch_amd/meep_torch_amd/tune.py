@@ -17,10 +17,14 @@ from . import _engine as E
 _CACHE = {}
 TUNE_STEPS = 24
 # variants from the smallest tile to the largest (mt_tiled_variants), and the
-# two timed on grids of more than one round.  Four steps or fewer do not repay
-# the tiled path's second buffer set.
+# two timed on grids of more than one round (of all shapes and the two-pass
+# path, ms per 200 steps: TM FP32 520 x 500 2.18 / 1.62 with 2 / 5, next 2.02;
+# 1500 x 1400 4.75 / 4.09, next 5.13; TE FP32 1500 x 1400 3.75 / 3.72, next
+# 4.47.  FP64 with 4 / 9: TM 520 x 500 3.05 / 2.20, next 2.36; 1500 x 1400 7.27 /
+# 7.19, next 8.11; TE 520 x 500 2.80 / 2.05, next 2.22; 2048^2 9.80 / 11.52, next
+# 11.35).  Four steps or fewer do not repay the tiled path's second buffer set.
 LADDER = {torch.float32: (8, 7, 9, 2, 5), torch.float64: (8, 7, 9, 2)}
-LARGE = {torch.float32: (2, 5), torch.float64: (2, 9)}
+LARGE = {torch.float32: (2, 5), torch.float64: (4, 9)}
 ROUND = 256                  # compute units: tiles that run side by side
 
 
@@ -75,8 +79,8 @@ def variant_for(mode, fields, coeffs, plan, monitors, k):
     v = one_round(ref.dtype, [tuple(ref.shape)])
     if v is not None:
         return v
-    if k < 2 * TUNE_STEPS:
-        return LARGE[ref.dtype][0]
+    if k < 2 * TUNE_STEPS:   # not timed; FP64: 16 x 64 x 2 wins from about 2^20 cells on
+        return LARGE[ref.dtype][ref.dtype == torch.float64 and ref.numel() < 2 ** 20]
     key = _key(mode, fields, monitors)
     if key not in _CACHE:
         _CACHE[key] = tune(mode, fields, coeffs, plan, monitors, cands=LARGE[ref.dtype])
