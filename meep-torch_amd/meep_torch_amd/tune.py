@@ -22,7 +22,7 @@ TUNE_STEPS = 24
 # 1500 x 1400 4.75 / 4.09, next 5.13; TE FP32 1500 x 1400 3.75 / 3.72, next
 # 4.47.  FP64 with 4 / 9: TM 520 x 500 3.05 / 2.20, next 2.36; 1500 x 1400 7.27 /
 # 7.19, next 8.11; TE 520 x 500 2.80 / 2.05, next 2.22; 2048^2 9.80 / 11.52, next
-# 11.35).  Four steps or fewer do not repay the tiled path's second buffer set.
+# 11.35).
 LADDER = {torch.float32: (8, 7, 9, 2, 5), torch.float64: (8, 7, 9, 2)}
 LARGE = {torch.float32: (2, 5), torch.float64: (4, 9)}
 ROUND = 256                  # compute units: tiles that run side by side
@@ -73,9 +73,15 @@ def variant_for(mode, fields, coeffs, plan, monitors, k):
     v = forced_variant()
     if v is not None:
         return v
-    if k <= 4:
-        return -1
     ref = fields["Ez"] if mode == "tm" else fields["Hz"]
+    if k <= 4:
+        # four steps or fewer do not repay the copy into a second buffer set,
+        # except the last of them on large FP32 grids (us, two-pass / 16 x 64 x 2
+        # tiles: TE 2048^2 k = 2 457 / 473, 3 517 / 482, 4 574 / 486; 1500 x 1400
+        # k = 4 437 / 423; TM 2048^2 k = 3 469 / 491, 4 521 / 507, 3000 x 2800
+        # k = 4 756 / 742; FP64 two-pass throughout)
+        paid = k - (3 if mode == "tm" else 2)
+        return 1 if ref.dtype == torch.float32 and paid * ref.numel() >= 2 ** 22 else -1
     v = one_round(ref.dtype, [tuple(ref.shape)])
     if v is not None:
         return v

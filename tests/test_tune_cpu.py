@@ -30,3 +30,14 @@ def test_large_grids(monkeypatch, mode):
 def test_grids_of_one_round(monkeypatch, mode):
     for shape, dtype, v in (((100, 60), F64, 8), ((256, 256), F32, 7), ((300, 300), F32, 9), ((500, 500), F32, 2)):
         assert _choice(monkeypatch, mode, shape, dtype, 400) == v
+
+
+def test_few_steps(monkeypatch):
+    c = lambda *a: _choice(monkeypatch, *a)
+    for mode in ("tm", "te"):
+        for k in (1, 2, 3, 4):
+            assert c(mode, (256, 256), F32, k) == c(mode, (2048, 2048), F64, k) == -1
+    assert [c("te", (2048, 2048), F32, k) for k in (1, 2, 3, 4)] == [-1, -1, 1, 1]
+    assert [c("te", (1500, 1400), F32, k) for k in (2, 3, 4)] == [-1, -1, 1]
+    assert [c("tm", (2048, 2048), F32, k) for k in (2, 3, 4)] == [-1, -1, 1]
+    assert c("tm", (1500, 1400), F32, 4) == -1
