@@ -355,7 +355,7 @@ int adj3_t(const mt_yee3d* d, const mt_yee3d_adj* a, const void* tape, const mt_
   const long long slot = (long long)(p.nx - 1) * p.ny * p.nz + (long long)p.nx * (p.ny - 1) * p.nz +
                          (long long)p.nx * p.ny * (p.nz - 1);
   const T* tp = static_cast<const T*>(tape);
-  const dim3 blk = block3(p.ny, p.nz), grd = grid3(blk, p.nx, p.ny, p.nz);
+  const dim3 blk = block3(p.ny, p.nz, sizeof(T)), grd = grid3(blk, p.nx, p.ny, p.nz);
   for (int s_ = k - 1; s_ >= 0; --s_) {
     const int t = step0 + s_;
     for (int m = 0; m < n_mons; ++m) {

@@ -6,6 +6,7 @@
 #include <string>
 
 #include "meep_fdtd.h"
+#include "schedule.h"
 
 namespace mt {
 
@@ -138,24 +139,10 @@ int monitors_sample(const MonitorPlan& mp, int slot, int t_rel, hipStream_t s);
 // Fold `n_filled` staged steps whose first global step index is t0 into the accumulators.
 int monitors_flush(const MonitorPlan& mp, int n_filled, int t0, double dt, hipStream_t s);
 
-// Workgroup (k, j) of the 3D per-cell kernels: rows along k (contiguous) of
-// equal length, at most 128 cells, and as many rows as 256 threads hold; waves
-// run on from one row into the next.  Whole 64-cell rows that fill a longer
-// axis exactly stay 64 x 4 below 384, as do rows of 52 to 63 cells, of which
-// 256 threads hold four in any case.  Wide rows read a row's cache lines in fewer
-// workgroups (no array starts its rows on a line) and leave few lanes idle.
-// Forward FP32 steps over 160 x 150 x nz (40 steps, 64 x 4 -> this): nz 40
-// 1831 -> 1624 us, 72 3172 -> 2389, 96 3308 -> 2840, 128 3692 -> 3442, 144
-// 4420 -> 4241, 300 7687 -> 7420; at 192 and 256 64 x 4 is as fast or faster
-// (4793 against 4808 with 96 x 2, 5662 against 5949 with 128 x 2); at 384 and
-// 512 128 x 2 is faster (8906 -> 8600, 11708 -> 11361; 384^3 45.99 -> 45.39
-// ms).  512 threads, and rows of 192 or more, gain nothing over both.
-constexpr int kBlock3 = 256;
-inline dim3 block3(int ny, int nz) {
-  const int m = (nz + 127) / 128, bx = (nz + m - 1) / m, by = kBlock3 / bx;
-  const bool rows64 = by == 4 || (m > 1 && nz % 64 == 0 && (nz % 128 || nz < 384));
-  if (rows64 || (ny + by - 1) / by > 65535) return dim3(64, 4, 1);
-  return dim3(bx, by, 1);
+// Workgroup (k, j) of the 3D per-cell kernels (rows3) and its grid.
+inline dim3 block3(int ny, int nz, size_t elem_size) {
+  const Rows3 r = rows3(ny, nz, elem_size == 8);
+  return dim3(r.bx, r.by, 1);
 }
 inline dim3 grid3(dim3 blk, int nx, int ny, int nz) {
   return dim3((nz + blk.x - 1) / blk.x, (ny + blk.y - 1) / blk.y, nx);

@@ -25,6 +25,41 @@ constexpr XcdItems xcd_items(int block, int grid, int total) {
 // forward and gradient over 400 steps: 13.14 -> 9.89 ms.
 constexpr int one_round_grid(int n) { return (n + 7) / 8 * 8; }
 
+// Rows of a workgroup of the 3D per-cell kernels: bx cells along k (contiguous)
+// by as many rows as 256 threads hold; waves run on from one row into the next.
+// Wide rows read a row's cache lines in fewer workgroups (no array starts its
+// rows on a line) and leave few lanes idle.
+//   nz <= 128      one row (rows of 52 to 63 cells as 64, four either way)
+//   nz <= 256      two equal rows; 64-cell rows where they fit exactly, and in
+//                  FP32 above 224, where they pad by less than an eighth
+//   above          128-cell rows; 64-cell rows at odd multiples of 64, above 384
+//                  where 128-cell rows pad by an eighth or more, and in FP64 up to 320
+// Forward steps over 160 x 150 x nz, 20 steps, us, 64 x 4 rows / this.  FP32: nz
+// 40 759 / 677, 72 1357 / 1008, 96 1416 / 1189, 128 1600 / 1466, 144 1936 /
+// 1852, 170 2159 / 2050, 200 2396 / 2396, 220 2481 / 2513, 257 2674 / 2587, 300 3387 /
+// 3129, 330 3913 / 3513, 384 3927 / 3783, 512 5271 / 5127, 640 6342 / 6099; FP64:
+// 72 2028 / 1477, 128 2457 / 2348, 200 5111 / 4590, 240 5493 / 4937, 330 7226 /
+// 6926, 512 10940 / 10038.  64-cell
+// rows where they stay: FP32 240 2445 (two rows 2572), 256, 448 4527 (four equal
+// rows 4876, 128-cell rows 4943), 704 6809 (7064), 576 equal; FP64 257 5476 (128-cell rows
+// 5552), 300 6210 (three equal rows 6781, 128-cell rows 6292), 448 8551 (9572,
+// 9753); 100 x 90 x 400 1713 (128-cell rows 1788).
+// 384^3 in FP32, timed in turn: 46.09 -> 45.88 ms for 40 steps.
+constexpr int kBlock3 = 256;
+struct Rows3 {
+  int bx, by;
+};
+constexpr Rows3 rows3(int ny, int nz, bool f64) {
+  int bx = nz <= 128 ? nz : nz <= 256 ? (nz + 1) / 2 : 128;
+  const int pad = (nz + 127) / 128 * 128 - nz;
+  if (nz % 128 == 64 || nz == 256 || (!f64 && nz > 224 && nz < 256) || (f64 && nz > 256 && nz <= 320) ||
+      (nz > 384 && 8 * pad >= nz + pad))
+    bx = nz > 128 ? 64 : bx;
+  const int by = kBlock3 / bx;
+  if (by == 4 || (ny + by - 1) / by > 65535) return Rows3{64, 4};
+  return Rows3{bx, by};
+}
+
 // Steps of each launch of a run of k steps: blocks of S steps (the monitors'
 // staging ring; S = k without monitors), NS per launch, the first launch of
 // several steps cut in two where the number would be odd, so that a run ends

@@ -1454,7 +1454,7 @@ int run3_tb2(const mt_yee3d* d, K3<T> p, const mt_source3d& sv, const double* co
   if (s_ < k) {   // odd count: the last step in place, two-pass
     void* const* A = in_alt ? B0 : A0;
     set_io(p, A, A);
-    const dim3 blk = block3(ny, nz), grd = grid3(blk, nx, ny, nz);
+    const dim3 blk = block3(ny, nz, sizeof(T)), grd = grid3(blk, nx, ny, nz);
     const T c = sv.kind ? static_cast<T>(coef[s_]) : T(0);
     hipLaunchKernelGGL((h3_kernel<T, false>), grd, blk, 0, s, p);
     hipLaunchKernelGGL((e3_kernel<T, false>), grd, blk, 0, s, p, sv, c, (T*)nullptr);
@@ -1528,7 +1528,7 @@ int run3_t(const mt_yee3d* d, const mt_source3d* src, const double* coef, const 
     }
     return run3_split<T, 4>(d, p, sv, coef, mp, step0, k, s);
   }
-  const dim3 blk = block3(p.ny, p.nz), grd = grid3(blk, p.nx, p.ny, p.nz);
+  const dim3 blk = block3(p.ny, p.nz, sizeof(T)), grd = grid3(blk, p.nx, p.ny, p.nz);
   int S = mp.stage_steps > 0 ? mp.stage_steps : 1;
   int filled = 0, first = step0;
   const long long e_cells = (long long)(p.nx - 1) * p.ny * p.nz + (long long)p.nx * (p.ny - 1) * p.nz +

@@ -34,6 +34,20 @@ int main() {
     if (one_round_grid(n) > 256) die("more workgroups than compute units", n, one_round_grid(n), 0);
   for (int grid : {8, 64, 256, 1024})
     for (int n : {1, 7, 9, 255, 257, 1000, 1025, 4099, 33000}) deal(grid, n, false);
+  // 3D rows: at most 256 threads, no lane of a whole column of workgroups idle
+  for (int f64 = 0; f64 < 2; ++f64)
+    for (int ny : {3, 40, 700, 200000, 262140})
+      for (int nz = 3; nz <= 1100; ++nz) {
+        const Rows3 r = rows3(ny, nz, f64);
+        if (r.bx < 1 || r.by < 1 || r.bx * r.by > kBlock3 || (ny + r.by - 1) / r.by > 65535) die("3D rows", ny, nz, f64);
+        if (ny < 1000 && (nz + r.bx - 1) / r.bx * r.bx - nz >= std::max(r.bx, 64)) die("3D rows idle", ny, nz, f64);
+      }
+  const int rows[][3] = {{40, 40, 40},   {56, 64, 64},   {72, 72, 72},    {128, 128, 128}, {144, 72, 72},
+                         {192, 64, 64},  {220, 110, 110}, {240, 64, 120}, {256, 64, 64},   {257, 128, 64},
+                         {300, 128, 64}, {330, 128, 128}, {384, 128, 128}, {400, 64, 64}, {448, 64, 64}, {500, 128, 128},
+                         {512, 128, 128}, {576, 64, 64}};
+  for (const auto& r : rows)
+    if (rows3(90, r[0], false).bx != r[1] || rows3(90, r[0], true).bx != r[2]) die("3D row rule", r[0], r[1], r[2]);
   for (int NS = 1; NS <= 8; ++NS)
     for (int S : {1, 2, 3, 5, 7, 8, 20, 64})
       for (int k = 1; k <= 210; ++k) {

@@ -11,7 +11,7 @@ from test_gpu_tb3d import _run
 pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not has_gpu(), reason="needs a HIP device")]
 
 
-@pytest.mark.parametrize("nz", [15, 63, 64, 65, 80, 127, 128, 129, 192, 257, 320, 384])
+@pytest.mark.parametrize("nz", [240, 300, 448, 15, 63, 64, 65, 80, 127, 128, 129, 192, 257, 320, 384])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64], ids=["f32", "f64"])
 def test_two_pass_rows_equal_split_step(nz, dtype):
     case = (19, 37, nz, 4, "mask", 7)
