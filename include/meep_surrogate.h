@@ -128,7 +128,9 @@ int mt_fno_fold(float* part, int Q, int n, float* out, void* stream);
 /* mt_pack_spectral for Ci = Co = C, and its per-mode transpose wp_t. */
 int mt_fno_pack(const float* wre, const float* wim, void* wp, void* wp_t, int C, int Mo, void* stream);
 
-/* y (C, R) = BF16 of x (R, C) transposed. */
+/* y_t (C, R) = BF16 of x (R, C) transposed, and y (R, C) = BF16 of x unless NULL. */
+int mt_cast_transpose_bf16(const float* x, void* y, void* y_t, int R, int C, void* stream);
+/* The same without y. */
 int mt_transpose_bf16(const float* x, void* y, int R, int C, void* stream);
 
 #ifdef __cplusplus

@@ -610,24 +610,51 @@ __global__ __launch_bounds__(256) void fold_kernel(float* part, int Q, int n, in
 
 // BF16 copies of the packed spectral weights (mt_pack_spectral), plain and
 // transposed per mode: the mixing kernel reads weight rows along its
-// reduction, forward from the transpose, backward from the plain form.
+// reduction, forward from the transpose, backward from the plain form.  The
+// weights lie along the modes, the copies along the channels: a block takes 32
+// modes of one input channel (blockIdx.z 0: two rows of every plain block) or
+// one output channel (1: two rows of the transposes) through LDS, so that both
+// sides are read and written in lines.  64 channels, 128 modes, per layer:
+// 17.8 us element by element, 9.5 this way (the plain copy alone 9.8); two
+// channels per store are no faster.
 __global__ __launch_bounds__(256) void pack_both_kernel(const float* wre, const float* wim, uint16_t* wp,
                                                         uint16_t* wt, int C, int Mo) {
-  const long long e = (long long)blockIdx.x * 256 + threadIdx.x, per = 4LL * C * C;
-  if (e >= per * Mo) return;
-  const int m = (int)(e / per), rem = (int)(e % per), k = rem / (2 * C), n = rem % (2 * C);
-  auto val = [&](int kk, int nn) {
-    const int pi = kk / C, i = kk % C, po = nn / C, o = nn % C;
-    const long long w = ((long long)i * C + o) * Mo + m;
-    return pi == po ? wre[w] : (pi == 0 ? wim[w] : -wim[w]);
-  };
-  wp[e] = bf(val(k, n));
-  wt[e] = bf(val(n, k));
+  constexpr int TM = 32, TA = 64;
+  __shared__ float re[TA][TM + 1], im[TA][TM + 1];
+  const int ch = blockIdx.x, m0 = blockIdx.y * TM;
+  const bool t = blockIdx.z;
+  uint16_t* out = t ? wt : wp;
+  for (int a0 = 0; a0 < C; a0 += TA) {
+    const int na = min(TA, C - a0), nm = min(TM, Mo - m0);
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < TA * TM / 256; ++it) {
+      const int x = threadIdx.x + it * 256, a = x / TM, m = x % TM;
+      if (a < na && m < nm) {
+        const long long w = ((long long)(t ? a0 + a : ch) * C + (t ? ch : a0 + a)) * Mo + m0 + m;
+        re[a][m] = wre[w];
+        im[a][m] = wim[w];
+      }
+    }
+    __syncthreads();
+    // rows r * C + ch, columns h * C + a: real where r == h, else +-imaginary
+    const int a = threadIdx.x % TA, h = threadIdx.x / TA & 1, r = threadIdx.x / (2 * TA);
+    const bool neg = t ? h > r : r > h;
+    if (a < na)
+      for (int m = 0; m < nm; ++m) {
+        const float v = r == h ? re[a][m] : neg ? -im[a][m] : im[a][m];
+        out[((long long)(m0 + m) * 2 * C + r * C + ch) * 2 * C + h * C + a0 + a] = bf(v);
+      }
+  }
 }
 
-__global__ void transpose_cast_kernel(const float* x, uint16_t* y, int R, int C) {
+// y = BF16 of x (R, C) where given, and yt its transpose
+__global__ void cast_transpose_kernel(const float* x, uint16_t* y, uint16_t* yt, int R, int C) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < R * C) y[(e % C) * R + e / C] = bf(x[e]);
+  if (e >= R * C) return;
+  const uint16_t v = bf(x[e]);
+  if (y) y[e] = v;
+  yt[(e % C) * R + e / C] = v;
 }
 
 bool al16(const void* p) { return p && (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -772,15 +799,20 @@ extern "C" int mt_fno_fold(float* part, int Q, int n, float* out, void* stream) 
 
 extern "C" int mt_fno_pack(const float* wre, const float* wim, void* wp, void* wp_t, int C, int Mo, void* stream) {
   if (!wre || !wim || !wp || !wp_t || C < 1 || Mo < 1) return fail(MT_EINVAL, "fno_pack: bad arguments");
-  const long long n = 4LL * C * C * Mo;
-  hipLaunchKernelGGL(pack_both_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), wre, wim, M16(wp), M16(wp_t), C, Mo);
+  if ((Mo + 31) / 32 > 65535) return fail(MT_EINVAL, "fno_pack: too many modes");
+  hipLaunchKernelGGL(pack_both_kernel, dim3(C, (Mo + 31) / 32, 2), dim3(256), 0, static_cast<hipStream_t>(stream), wre,
+                     wim, M16(wp), M16(wp_t), C, Mo);
   return check_launch("fno_pack");
 }
 
+extern "C" int mt_cast_transpose_bf16(const float* x, void* y, void* y_t, int R, int C, void* stream) {
+  if (!x || !y_t || R < 1 || C < 1) return fail(MT_EINVAL, "cast_transpose_bf16: bad arguments");
+  hipLaunchKernelGGL(cast_transpose_kernel, dim3((R * C + 255) / 256), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), x, M16(y), M16(y_t), R, C);
+  return check_launch("cast_transpose_bf16");
+}
+
 extern "C" int mt_transpose_bf16(const float* x, void* y, int R, int C, void* stream) {
-  if (!x || !y || R < 1 || C < 1) return fail(MT_EINVAL, "transpose_bf16: bad arguments");
-  hipLaunchKernelGGL(transpose_cast_kernel, dim3((R * C + 255) / 256), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), x, M16(y), R, C);
-  return check_launch("transpose_bf16");
+  if (!y) return fail(MT_EINVAL, "transpose_bf16: bad arguments");
+  return mt_cast_transpose_bf16(x, nullptr, y, R, C, stream);
 }

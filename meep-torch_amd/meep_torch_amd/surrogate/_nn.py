@@ -46,9 +46,9 @@ def lib():
     L.mt_fno_head_back.argtypes = [V] * 14 + [I, I, I, I, V]
     L.mt_fno_fold.argtypes = [V, I, I, V, V]
     L.mt_fno_pack.argtypes = [V, V, V, V, I, I, V]
-    L.mt_transpose_bf16.argtypes = [V, V, I, I, V]
+    L.mt_cast_transpose_bf16.argtypes = [V, V, V, I, I, V]
     for n in ("mt_fno_lift", "mt_fno_lift_back", "mt_fno_dft", "mt_fno_mix", "mt_fno_out", "mt_fno_out_back",
-              "mt_fno_head", "mt_fno_head_back", "mt_fno_fold", "mt_fno_pack", "mt_transpose_bf16"):
+              "mt_fno_head", "mt_fno_head_back", "mt_fno_fold", "mt_fno_pack", "mt_cast_transpose_bf16"):
         getattr(L, n).restype = c_int
     for n in ("mt_gemm_bf16", "mt_cast_bf16", "mt_bias_act", "mt_act_grad", "mt_channel_sum", "mt_row_sum",
               "mt_pack_spectral", "mt_unpack_spectral_grad", "mt_adam"):
@@ -145,6 +145,14 @@ def row_sum(x, out, rows, P, scale=1.0):
 
 def pack_spectral(wre, wim, wp, Ci, Co, Mo):
     E.check(lib().mt_pack_spectral(_p(wre), _p(wim), _p(wp), Ci, Co, Mo, E.stream_handle()), "mt_pack_spectral")
+
+
+def pack_both(wre, wim, wp, wpt, C, Mo):
+    E.check(lib().mt_fno_pack(_p(wre), _p(wim), _p(wp), _p(wpt), C, Mo, E.stream_handle()), "mt_fno_pack")
+
+
+def cast_transpose(x, y, yt, R, C):
+    E.check(lib().mt_cast_transpose_bf16(_p(x), _p(y), _p(yt), R, C, E.stream_handle()), "mt_cast_transpose_bf16")
 
 
 def unpack_spectral_grad(dwp, dwre, dwim, Ci, Co, Mo):

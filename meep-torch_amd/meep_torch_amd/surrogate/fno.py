@@ -155,25 +155,28 @@ class SpectralOperator:
     def sync_weights(self):
         """Refresh the BF16 weight copies from `params` (after init, load or an
         optimizer step)."""
-        C, Mo = self.C, self.Mo
+        C, Mo, bf = self.C, self.Mo, torch.bfloat16
+
+        W, p = self._wbf, self.p
+        if not W:
+            for name in ["lift_w", "q_w", "o_w"] + [f"w{l}" for l in range(self.L)]:
+                W[name] = torch.empty(p[name].shape, dtype=bf, device=self.device)
+                if self.fused and name not in ("lift_w", "o_w"):   # also the transpose, which the fused passes read
+                    W[name + "T"] = torch.empty(p[name].shape[::-1], dtype=bf, device=self.device)
+            for l in range(self.L):
+                for name in (f"wp{l}", f"wp{l}T")[:1 + self.fused]:
+                    W[name] = torch.empty((Mo, 2 * C, 2 * C), dtype=bf, device=self.device)
         for name in ["lift_w", "q_w", "o_w"] + [f"w{l}" for l in range(self.L)]:
-            t = self.p[name]
-            if name not in self._wbf:
-                self._wbf[name] = torch.empty(t.shape, dtype=torch.bfloat16, device=self.device)
-            _nn.cast_bf16(t, self._wbf[name])
-        if self.fused:   # also the transposes that the fused passes read along their reductions
-            for name, R, Q in [("q_w", self.H, C)] + [(f"w{l}", C, C) for l in range(self.L)]:
-                t = self._wbf.setdefault(name + "T", torch.empty((Q, R), dtype=torch.bfloat16, device=self.device))
-                _nn.fno("transpose_bf16", self.p[name], t, R, Q)
+            t = p[name]
+            if name + "T" in W:
+                _nn.cast_transpose(t, W[name], W[name + "T"], *t.shape)
+            else:
+                _nn.cast_bf16(t, W[name])
         for l in range(self.L):
-            key = f"wp{l}"
-            if key not in self._wbf:
-                self._wbf[key] = torch.empty((Mo, 2 * C, 2 * C), dtype=torch.bfloat16, device=self.device)
             if self.fused:
-                t = self._wbf.setdefault(key + "T", torch.empty_like(self._wbf[key]))
-                _nn.fno("fno_pack", self.p[f"s{l}_re"], self.p[f"s{l}_im"], self._wbf[key], t, C, Mo)
-                continue
-            _nn.pack_spectral(self.p[f"s{l}_re"], self.p[f"s{l}_im"], self._wbf[key], C, C, Mo)
+                _nn.pack_both(p[f"s{l}_re"], p[f"s{l}_im"], W[f"wp{l}"], W[f"wp{l}T"], C, Mo)
+            else:
+                _nn.pack_spectral(p[f"s{l}_re"], p[f"s{l}_im"], W[f"wp{l}"], C, C, Mo)
 
     def state_dict(self):
         return {"params": self.params.detach().cpu().clone(), "step": self.step_count,
