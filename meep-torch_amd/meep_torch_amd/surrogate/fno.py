@@ -95,19 +95,31 @@ class SpectralOperator:
         self.p, self.g = self._views(self.params), self._views(self.grads)
         self.init_params(seed)
         F, G = dft_bases(n, self.mx, self.my)
-        self.F = self._bf(F)                        # (2Mo, P)
-        self.FT = self._bf(np.ascontiguousarray(F.T))  # (P, 2Mo)
-        self.G = self._bf(G)
-        self.GT = self._bf(np.ascontiguousarray(G.T))
+        self.F, self.G = self._bf(F), self._bf(G)   # (2Mo, P)
+        self._rows = {}
         self.ws = _nn.Workspace(self.device)
         self._wbf = {}
         # the fused passes' size (spectral.hip); their 128-bit loads need rows
         # of whole 16-point groups
         self.fused = (self.C == 64 and self.Mo == 128 and self.H == 128 and self.in_ch == 3 and self.P % 16 == 0)
         if self.fused:
-            self.GTf, self.FTf = self._fragments(self.GT), self._fragments(self.FT)
+            self.GTf, self.FTf = self._fragments(self.G.t()), self._fragments(self.F.t())
         self.sync_weights()
         self._buf = {}
+
+    @property
+    def FT(self):
+        """(P, 2Mo): F transposed for the general kernels, kept from its first use."""
+        return self._basis_rows("F", self.F)
+
+    @property
+    def GT(self):
+        return self._basis_rows("G", self.G)
+
+    def _basis_rows(self, name, basis):
+        if name not in self._rows:
+            self._rows[name] = basis.t().contiguous()
+        return self._rows[name]
 
     @staticmethod
     def _fragments(t):
@@ -116,7 +128,7 @@ class SpectralOperator:
         K, then lane = 32 * half + point with 8 values each."""
         P, K = t.shape
         pad = -P % 128
-        t = torch.cat([t, t.new_zeros(pad, K)]) if pad else t
+        t = torch.cat([t, t.new_zeros(pad, K)]) if pad else t.contiguous()
         return t.view(-1, 32, K // 16, 2, 8).permute(0, 2, 3, 1, 4).contiguous()
 
     # ---- parameters -------------------------------------------------------

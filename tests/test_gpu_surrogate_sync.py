@@ -40,3 +40,16 @@ def test_refresh_allocates_nothing():
     before = count()
     net.sync_weights()
     assert count() == before
+
+
+def test_general_bases_only_where_used():
+    """The row-major bases of the general kernels are made on first use: a
+    network on the fused passes holds the bases once and the fragments."""
+    from meep_torch_amd.surrogate.fno import SpectralOperator, dft_bases
+    net = SpectralOperator(n=16, n_out=5)
+    net.backward(torch.ones_like(net.forward(torch.rand(2, 16, 16, device="cuda"))))
+    assert net.fused and not any(k in vars(net) for k in ("FT", "GT")) and not net._rows
+    F, G = dft_bases(16, 16, 8)
+    for got, want in ((net.FT, F), (net.GT, G)):
+        assert got.is_contiguous() and torch.equal(got, torch.from_numpy(want.T.copy()).float().bfloat16().cuda())
+    assert net.FT is net.FT
