@@ -134,11 +134,7 @@ TmTiled<T> tiled_of(const mt_tm2d* d, const mt_source2d* src, const void* coef_t
   p.hx = pml_of<T>(d->hx);
   p.ex = pml_of<T>(d->ex);
   p.ey = pml_of<T>(d->ey);
-  const int joff = d->y_pmc ? 0 : 1;
-  p.in_i0 = std::max(d->hx.lo_end, d->ex.lo_end + 1) + 1;
-  p.in_i1 = std::min(d->hx.hi_begin, d->ex.hi_begin + 1) - 1;
-  p.in_j0 = std::max(d->hy.lo_end, d->ey.lo_end + joff) + 1;
-  p.in_j1 = std::min(d->hy.hi_begin, d->ey.hi_begin + joff) - 1;
+  tm_interior(d, &p.in_i0, &p.in_i1, &p.in_j0, &p.in_j1);
   p.map = tiled_map(variant, d->dtype, d->nx, d->ny, p.in_i0, p.in_i1, p.in_j0, p.in_j1);
   T* A[8] = {static_cast<T*>(d->Ez), static_cast<T*>(d->Dz), static_cast<T*>(d->Hx), static_cast<T*>(d->Hy),
              static_cast<T*>(d->psi_Ezy), static_cast<T*>(d->psi_Ezx), static_cast<T*>(d->psi_Hyx),

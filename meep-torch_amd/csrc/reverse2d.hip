@@ -433,8 +433,6 @@ int with_shape(int variant, F f) {
   }
 }
 
-constexpr int kOneRound = 256;   // tiles up to which one launch covers interior and ring (tiled2d.hip)
-
 template <typename T>
 struct RevLaunch {
   TmRev<T> p;
@@ -540,11 +538,7 @@ TmRev<T> make_rev(const mt_tm2d* d, const mt_tm2d_adj* r, const mt_tm2d_adj* w, 
   p.hx = pml_of<T>(d->hx);
   p.ex = pml_of<T>(d->ex);
   p.ey = pml_of<T>(d->ey);
-  const int joff = d->y_pmc ? 0 : 1;
-  p.in_i0 = std::max(d->hx.lo_end, d->ex.lo_end + 1) + 1;
-  p.in_i1 = std::min(d->hx.hi_begin, d->ex.hi_begin + 1) - 1;
-  p.in_j0 = std::max(d->hy.lo_end, d->ey.lo_end + joff) + 1;
-  p.in_j1 = std::min(d->hy.hi_begin, d->ey.hi_begin + joff) - 1;
+  tm_interior(d, &p.in_i0, &p.in_i1, &p.in_j0, &p.in_j1);
   p.Ez = static_cast<const T*>(r->aEz), p.Dz = static_cast<const T*>(r->aDz);
   p.Hx = static_cast<const T*>(r->aHx), p.Hy = static_cast<const T*>(r->aHy);
   p.pEzy = static_cast<const T*>(r->apsi_Ezy), p.pEzx = static_cast<const T*>(r->apsi_Ezx);

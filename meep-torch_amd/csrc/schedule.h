@@ -18,6 +18,8 @@ constexpr XcdItems xcd_items(int block, int grid, int total) {
   const int x = block & 7, chunk = (total + 7) >> 3, end = (x + 1) * chunk;
   return XcdItems{x * chunk + (block >> 3), end < total ? end : total, (grid - x + 7) >> 3};
 }
+constexpr int kOneRound = 256;   // compute units: tiles that run side by side (tune.py's ROUND)
+
 // Workgroups of a launch over n items in which no workgroup takes two: every
 // XCD gets as many as its range has items (with n workgroups some XCDs have
 // one fewer than items, and the launch lasts two tiles instead of one); those

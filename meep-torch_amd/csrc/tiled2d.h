@@ -95,6 +95,15 @@ constexpr int kAvgVariant = 1000;
 bool taps_avg_d(const mt_monitor* mons, int n);
 int tiled_variant_steps(int variant, int dtype);
 
+// Cells whose tiles carry no CPML psi: rows [i0, i1) x columns [j0, j1).
+inline void tm_interior(const mt_tm2d* d, int* i0, int* i1, int* j0, int* j1) {
+  const int joff = d->y_pmc ? 0 : 1;
+  *i0 = std::max(d->hx.lo_end, d->ex.lo_end + 1) + 1;
+  *i1 = std::min(d->hx.hi_begin, d->ex.hi_begin + 1) - 1;
+  *j0 = std::max(d->hy.lo_end, d->ey.lo_end + joff) + 1;
+  *j1 = std::min(d->hy.hi_begin, d->ey.hi_begin + joff) - 1;
+}
+
 // Build the tap set of a tiled launch from the monitor plan; false if some
 // term has no semantic form (then the per-half-step path must be used).
 bool build_taps(const MonitorPlan& mp, int slot0, int t_rel0, int elem_size, TapSet* out);

@@ -676,8 +676,6 @@ tm_batch_in2(const TmBatchVar<T>* vars, const int* pre_in, const int* pre_ring, 
 // workgroups per CU).  The interior (or common) launch is the one the kernel
 // timing hook measures, its cell-steps the cells of its tiles times the
 // substeps.
-constexpr int kOneRound = 256;
-
 template <typename KA, typename K1, typename K2>
 void launch_tiles(const TileMap& m, KA kall, K1 kin, K2 kpml, hipStream_t s, long long tile_cells, int nsub) {
   const int n_in = (m.r1 - m.r0) * (m.c1 - m.c0), n = m.R * m.C, n_ring = n - n_in;

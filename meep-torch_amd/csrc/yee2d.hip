@@ -604,15 +604,7 @@ int te_run_t(const mt_te2d* d, const mt_source2d* src, const double* coef, const
   return MT_OK;
 }
 
-// Cells whose tiles carry no CPML psi: rows [i0, i1) x columns [j0, j1).
-void tm_interior(const mt_tm2d* d, int* i0, int* i1, int* j0, int* j1) {
-  const int joff = d->y_pmc ? 0 : 1;
-  *i0 = std::max(d->hx.lo_end, d->ex.lo_end + 1) + 1;
-  *i1 = std::min(d->hx.hi_begin, d->ex.hi_begin + 1) - 1;
-  *j0 = std::max(d->hy.lo_end, d->ey.lo_end + joff) + 1;
-  *j1 = std::min(d->hy.hi_begin, d->ey.hi_begin + joff) - 1;
-}
-
+// The same of a TE grid.
 void te_interior(const mt_te2d* d, int* i0, int* i1, int* j0, int* j1) {
   *i0 = std::max(d->hx.lo_end, d->ex.lo_end + 1) + 1;
   *i1 = std::min(d->hx.hi_begin, d->ex.hi_begin + 1) - 1;

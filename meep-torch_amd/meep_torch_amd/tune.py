@@ -25,7 +25,7 @@ TUNE_STEPS = 24
 # 11.35).
 LADDER = {torch.float32: (8, 7, 9, 2, 5), torch.float64: (8, 7, 9, 2)}
 LARGE = {torch.float32: (2, 5), torch.float64: (4, 9)}
-ROUND = 256                  # compute units: tiles that run side by side
+ROUND = 256                  # compute units: tiles that run side by side (kOneRound, schedule.h)
 
 
 def variants(dtype):
