@@ -105,16 +105,17 @@ def test_batched_gradient_central_fd():
     assert float(eps_b[0].grad.abs().max()) == 0.0
 
 
-BIG = [(336, 310), (392, 448)]
+BIG = [(700, 720), (520, 610)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_batched_interior_tiles_match_two_pass(dtype, monkeypatch):
-    """Grids large enough that the batched launch's interior-tile kernel
-    (tm_batch<..., PML = false>, the FP32 32 x 64 x 4-step tile the C4 design
-    loop runs) carries about half the cells or more: spectra bit-identical to the two-pass
-    per-half-step path, and the batched gradient equal to the single-problem
-    adjoint's."""
+    """A batch of more than one round of tiles, so that interior and ring tiles
+    have launches of their own (FP32: the 32 x 64 x 4-step tile large batches
+    run) and interior tiles carry half the cells or more: spectra
+    bit-identical to the two-pass per-half-step path, the gradient bit for bit
+    that of the three transpose passes and equal to the single-problem
+    step-by-step adjoint's."""
     from meep_torch_amd.batch import BatchedTM
     from meep_torch_amd.core import engine2d
     from meep_torch_amd.core.monitors import FluxMonitorTM
@@ -126,13 +127,19 @@ def test_batched_interior_tiles_match_two_pass(dtype, monkeypatch):
         mon = FluxMonitorTM(g, [0.8, 1.0, 1.2], x_normal=True, idx=80, lo=9, hi=ny - 9)
         probs.append((g, m, src, mon, eps))
     bt = BatchedTM([(m, src, [mon]) for (g, m, src, mon, eps) in probs], N_STEPS, checkpoint_every=CK)
-    for (g, m, src, mon, eps), (nx, ny) in zip(probs, BIG):
-        n_in, n_ring = engine2d.tile_counts("tm", nx, ny, m, dtype, bt.variant)
-        assert n_in >= 25 and n_ring > 0, (n_in, n_ring)   # interior tiles: about half the grid or more
+    counts = [engine2d.tile_counts("tm", nx, ny, p[1], dtype, bt.variant) for p, (nx, ny) in zip(probs, BIG)]
+    assert sum(map(sum, counts)) > 256 and all(n_in >= n_ring > 0 for n_in, n_ring in counts), counts
+    assert dtype == torch.float64 or bt.variant == 5
     eps_b = [p[4].clone().requires_grad_(True) for p in probs]
     out = bt.apply(eps_b)
     J = sum(mon.flux(o[0], 0.05).sum() for (_, _, _, mon, _), o in zip(probs, out))
     J.backward()
+    assert bt._adj["fused"]
+    passes = BatchedTM([(m, src, [mon]) for (g, m, src, mon, eps) in probs], N_STEPS, checkpoint_every=CK,
+                       fused_adjoint=False)
+    eps_p = [p[4].clone().requires_grad_(True) for p in probs]
+    sum(mon.flux(o[0], 0.05).sum() for (_, _, _, mon, _), o in zip(probs, passes.apply(eps_p))).backward()
+    assert all(torch.equal(a.grad, b.grad) for a, b in zip(eps_b, eps_p))
     monkeypatch.setenv("MEEP_TORCH_AMD_VARIANT", "-1")
     for (g, m, src, mon, eps), o, eb in zip(probs, out, eps_b):
         e1 = eps.clone().requires_grad_(True)
@@ -142,6 +149,39 @@ def test_batched_interior_tiles_match_two_pass(dtype, monkeypatch):
         mon.flux(ref, 0.05).sum().backward()
         rel = float((eb.grad - e1.grad).norm() / e1.grad.norm())
         assert rel <= (1e-12 if dtype == torch.float64 else 1e-6), rel
+
+
+def test_workgroups_with_several_tiles(monkeypatch):
+    """More interior tiles than workgroups: a workgroup walks several items,
+    of several variants."""
+    from meep_torch_amd.batch import BatchedTM
+    from meep_torch_amd.core import engine2d
+    from meep_torch_amd.core.monitors import FluxMonitorTM
+    from meep_torch_amd.core.run import run_tm
+    from meep_torch_amd.core.stepper_tm import init_tm_state
+    sizes, n, ck = [(900, 1010), (930, 1000), (880, 1090), (910, 980)], 30, 15
+    probs = []
+    for i, (nx, ny) in enumerate(sizes):
+        g, m, src, _, eps = _problem(nx, ny, torch.float32, 80 + i)
+        probs.append((g, m, src, FluxMonitorTM(g, [0.8, 1.2], x_normal=True, idx=17, lo=9, hi=ny - 9), eps))
+    grads = []
+    for fused in (True, False):
+        bt = BatchedTM([(m, src, [mon]) for (g, m, src, mon, eps) in probs], n, checkpoint_every=ck,
+                       fused_adjoint=fused)
+        inner = sum(engine2d.tile_counts("tm", nx, ny, p[1], torch.float32, bt.variant)[0]
+                    for p, (nx, ny) in zip(probs, sizes))
+        assert inner > 4 * torch.cuda.get_device_properties(0).multi_processor_count
+        eps_b = [p[4].clone().requires_grad_(True) for p in probs]
+        out = bt.apply(eps_b)
+        sum((o[0] ** 2).sum() for o in out).backward()
+        assert bt._adj["fused"] == fused
+        grads.append([e.grad for e in eps_b])
+    for a, b in zip(*grads):
+        assert float(a.abs().max()) > 0 and torch.equal(a, b)
+    monkeypatch.setenv("MEEP_TORCH_AMD_VARIANT", "-1")
+    for (g, m, src, mon, eps), o in zip(probs, out):
+        _, (acc,) = run_tm(init_tm_state(g), m._replace(eps_inf=eps), n, source=src, monitors=[mon], checkpoint_every=ck)
+        assert float(acc.abs().max()) > 0 and torch.equal(o[0].detach(), acc)
 
 
 def test_adjoint_graph_replays_match_eager():
@@ -180,11 +220,10 @@ def test_adjoint_graph_replays_match_eager():
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("ck", [CK, 75])
 def test_fused_adjoint_step_equals_three_passes(dtype, ck):
-    """The fused reverse step (one tiled pass per step, two cotangent sets,
+    """The tiled reverse launches (several steps each, two cotangent sets,
     transposed differences in LDS) against the three transpose passes: eps
-    gradients bit for bit, with segments of an even (100) and an odd (75,
-    the result copied back from the second set) number of steps, on grids
-    that end in partial tiles in both directions."""
+    gradients bit for bit, with segments of an even (100) and an odd (75)
+    number of steps, on grids that end in partial tiles in both directions."""
     from meep_torch_amd.batch import BatchedTM
     sizes = SIZES + [(83, 131)]
     probs = [_problem(nx, ny, dtype, 60 + i) for i, (nx, ny) in enumerate(sizes)]

@@ -1,7 +1,8 @@
-"""Runs of tiled launches end in the buffers they began in: step counts that
-need one launch, an even and an odd number of them, a last launch of one step
-and a staging block that ends inside the run, bit-identical to the two-pass
-path."""
+"""Runs of any number of tiled launches are bit-identical to the two-pass path:
+step counts that need one launch, an even and an odd number of them, a last
+launch of one step, a staging block that ends inside the run, and staging blocks
+shorter than a launch.  (That launches come in an even number, so that runs end
+in the buffers they began in, is checked in test_schedule_cpu.py.)"""
 import pytest
 import torch
 
@@ -20,3 +21,13 @@ def test_any_step_count_matches_two_pass(mode, variant, k):
                     _run(mode, torch.float32, -1, (65, 50), k, 6)):
         assert torch.equal(a, b)
 
+
+@pytest.mark.parametrize("S", [1, 3, 7])
+@pytest.mark.parametrize("variant", [2, 7, 8])
+@pytest.mark.parametrize("mode", ["tm", "te"])
+def test_short_staging_blocks(mode, variant, S, monkeypatch):
+    from meep_torch_amd.core import engine2d
+    monkeypatch.setattr(engine2d, "STAGE_STEPS", S)
+    for a, b in zip(_run(mode, torch.float32, variant, (65, 50), 23, 6),
+                    _run(mode, torch.float32, -1, (65, 50), 23, 6)):
+        assert torch.equal(a, b)

@@ -2,7 +2,8 @@
 per-step passes (mt_tm2d_adjoint), bit for bit: every cotangent, eps gradient,
 x and y lines, whole-field and D monitors, probes, odd and even launch counts,
 staging blocks shorter than the sweep, one- and two-step sweeps, tiles of
-every shape on grids below, at and above a multiple of the tile."""
+every shape on grids below, at and above a multiple of the tile, in the common
+launch of a one-round grid and in the interior and ring launches of a larger one."""
 import ctypes
 
 import pytest
@@ -69,7 +70,7 @@ def _sweeps(dtype, size, npml, k, variant, S, y_pmc=False):
 
 
 @pytest.mark.parametrize("size,npml,k,S", [((5, 7), 1, 1, 4), ((33, 31), 4, 2, 64), ((64, 96), 6, 19, 7),
-                                           ((130, 71), 8, 30, 64), ((210, 190), 7, 9, 3)])
+                                           ((130, 71), 8, 30, 64), ((210, 190), 7, 9, 3), ((530, 1060), 20, 6, 4)])
 @pytest.mark.parametrize("variant", [2, 5, 7, 8, 9])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_tiled_reverse_matches_per_step_passes(dtype, variant, size, npml, k, S):
