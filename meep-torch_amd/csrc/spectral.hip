@@ -24,13 +24,17 @@
 //               operand without leaving registers), channel sums
 // BF16 operands, FP32 accumulation (v_mfma_f32_32x32x16_bf16); biases, GELU,
 // pre-activations and sums FP32, as in the general path.  Partial sums are
-// folded in a fixed order, so results do not depend on scheduling.
-// Batch 64 of 128^2 points, 4 layers, forward + backward + optimizer:
-// 10.77 -> 3.02 ms; one sample's forward and input gradient 0.89 -> 0.45 ms.
-// Per launch at that batch: dft 60 us, out 184 us, backward out 242 us, head
-// backward 564 us (134 MB of BF16 and 268 MB of FP32 activations are 26 and
-// 52 us at the rate of a large copy); the vector work of GELU and of the
-// operand conversions bounds what is left.
+// folded in a fixed order, so results do not depend on scheduling; the order
+// does depend on a sample's place in its batch (dft's first step), so the same
+// sample at two places differs by FP32 rounding and what BF16 makes of it.
+// Batch 64 of 128^2 points, 4 layers, forward + every gradient: 10.77 -> 3.02
+// ms; one sample's forward and input gradient 0.89 -> 0.45 ms.
+// Per launch at that batch: dft 61 us, with the weight gradient 107, out 185 us,
+// backward out 242 us, head forward 157 us, head backward 550 us (134 MB of BF16
+// and 268 MB of FP32 activations are 26 and 52 us at the rate of a large copy).
+// The vector work of GELU and of the operand conversions bounds them, and the
+// head backward with gradients its registers too: 256 VGPRs and 47 spilled (192 B
+// of scratch per lane) beside 32 persistent accumulators.
 //
 // MFMA fragments (32x32x16): lane l holds A row / B column l & 31, reduction
 // elements 8 (l >> 5) .. + 7; result column l & 31, rows 8 (r >> 2) +

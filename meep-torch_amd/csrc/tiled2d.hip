@@ -601,8 +601,8 @@ __global__ __launch_bounds__((Shape<TX, TY, NS, kMaxTm>::BLK)) void tm_tiled(TmT
 
 // FP32 interior tiles held to 64 VGPRs (eight waves per SIMD): two
 // 1024-thread workgroups fit a CU (their LDS allows it), so one hides the
-// other's barrier and load latency.  Ring tiles (CPML psi) and FP64 keep the
-// plain bound.
+// other's barrier and load latency (the 32 x 64 shapes spill 9 VGPRs, 40 B of
+// scratch, for it).  Ring tiles (CPML psi) and FP64 keep the plain bound.
 template <typename T, int TX, int TY, int NS>
 __global__ __launch_bounds__((Shape<TX, TY, NS, kMaxTm>::BLK)) __attribute__((amdgpu_waves_per_eu(8, 8))) void
 tm_tiled_in2(TmTiled<T> p, TapSet taps, int nsub, int tape_s0) {
@@ -766,7 +766,10 @@ TileMap map_for(int nx, int ny, int in_i0, int in_i1, int in_j0, int in_j1) {
 
 // Tile-shape variants (index = variant id), (TX, TY, NS): owned rows, owned
 // columns, Yee steps per launch.  FP64 tiles are smaller so that registers
-// and LDS fit one workgroup.  Variants 0-6 are for grids that fill the chip;
+// and LDS fit one workgroup.  Variants 0-6 are for grids that fill the chip
+// (tune.py chooses 2 and 5 in FP32, 2 and 4 in FP64, 1 for a few steps on large
+// grids; 0, 3 and 6, and 1 and 5 of FP64, only callers that name them: variant
+// arguments, MEEP_TORCH_AMD_VARIANT, tune());
 // 7 on are for grids that do not: there a launch lasts as long as one tile
 // (VALU issue of the tile's cells on one CU, about 0.3 us per half-step and
 // 1000 cells, over about 6 us of launch, load and store latency), so the
